@@ -298,8 +298,10 @@ MI355X_API int mi355x_gemv_batched(mi355x_ctx *ctx, int type, const void *W, int
 /* Allocation-free form of mi355x_gemv_batched, for callers that cannot call
  * hipMalloc (code under HIP graph capture, tight serving loops, harnesses
  * that forbid it).  No counterpart in the reference.  Same arguments and the
- * same outputs, bit for bit; the K-split batched form keeps its activation
- * tiles in the library's static device scratch of
+ * same outputs, bit for bit; the matrix-core form converts activations in
+ * each workgroup and takes the segments of K one after another; the K-split
+ * batched form keeps its activation tiles in the library's static device
+ * scratch of
  * MI355X_NOALLOC_SCRATCH_BYTES (336 KiB per device, held until the process
  * ends; enough for 8 activations of K = 16384 per pass, the most the form
  * stages) instead of a context buffer grown with hipMalloc.  Every call on

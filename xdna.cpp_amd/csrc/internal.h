@@ -28,6 +28,10 @@ struct mi355x_ctx {
     // demand, freed with the context)
     void *mbtiles = nullptr;
     size_t mbtiles_bytes = 0;
+    // activation planes and K-segment partials of a matrix-core batched call
+    // (grown on demand, freed with the context)
+    void *gemm_buf = nullptr;
+    size_t gemm_bytes = 0;
     // device address of the library's static scratch on this device
     // (allocation-free entry point)
     void *scratch = nullptr;
@@ -35,6 +39,9 @@ struct mi355x_ctx {
     void *iq3xxs_grid = nullptr;
     void *iq2s_grid = nullptr;
     uint64_t grids_version = 0;
+    // largest magnitude of each grid
+    int iq3xxs_max = 0;
+    int iq2s_max = 0;
     // tuning / numerics options (mi355x_ctx_set_option)
     int kernel_variant = MI355X_VARIANT_AUTO;
     int rows_override = 0;
@@ -117,6 +124,12 @@ int launch_gemv_q4_0_mb(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
 // current); resolved once per device with hipGetSymbolAddress.
 int resolve_scratch(int device, void **out);
 size_t scratch_bytes();
+// Matrix-core form of a batched call (any weight type): whether it takes M
+// activation rows of `a`, and its launches.  noalloc: no context buffer; the
+// same outputs bit for bit.
+bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M);
+int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int64_t M,
+                        bool noalloc);
 // Several Q4_0 matrices that share the activation row x as one launch of
 // the pipelined form (*launched = false where that form does not apply: the
 // caller launches each matrix on its own).

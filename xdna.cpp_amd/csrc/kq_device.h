@@ -82,6 +82,33 @@ __device__ __forceinline__ u32x3 ld96(const Row &r, uint32_t off) {
     return __builtin_amdgcn_raw_buffer_load_b96(r.rsrc, static_cast<int>(off), 0, kNonTemporal);
 }
 
+// A view in which every lane reads a row of its own: one buffer over a run of
+// consecutive rows, the lane's row starting `base` bytes into it.  Its loads
+// are cached (several workgroups read the same weights), unlike Row's.
+struct LaneRow {
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t base;
+    uint32_t P[5];  // as Row::P, of the lane's row
+};
+__device__ __forceinline__ u32x4 ld128(const LaneRow &r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r.rsrc, static_cast<int>(r.base + off), 0, 0);
+}
+__device__ __forceinline__ u32x3 ld96(const LaneRow &r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b96(r.rsrc, static_cast<int>(r.base + off), 0, 0);
+}
+__device__ __forceinline__ u32x2 ld64(const LaneRow &r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b64(r.rsrc, static_cast<int>(r.base + off), 0, 0);
+}
+__device__ __forceinline__ uint32_t ld32(const LaneRow &r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r.rsrc, static_cast<int>(r.base + off), 0, 0);
+}
+__device__ __forceinline__ uint32_t ld16(const LaneRow &r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b16(r.rsrc, static_cast<int>(r.base + off), 0, 0);
+}
+__device__ __forceinline__ uint32_t ld8(const LaneRow &r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b8(r.rsrc, static_cast<int>(r.base + off), 0, 0);
+}
+
 // Buffer view of one row; rows at or past `lim` get an empty range.
 template <int TYPE>
 __device__ __forceinline__ Row make_row_pl(const KqArgs &a, int64_t row, int64_t lim) {
@@ -108,7 +135,8 @@ __device__ __forceinline__ Row make_row_pl(const KqArgs &a, int64_t row, int64_t
 struct GPos {
     uint32_t base, g, bl, m, d;
 };
-__device__ __forceinline__ GPos gpos(const Row &r, int bb, uint32_t b, int s) {
+template <class RowT>
+__device__ __forceinline__ GPos gpos(const RowT &r, int bb, uint32_t b, int s) {
     const uint32_t B = r.P[0];
     const bool flipped = r.P[1] != 0;
     const uint32_t t = b >> 3;
@@ -270,7 +298,8 @@ struct Kq<MI355X_TYPE_Q4_K> {
     struct Regs {
         u32x4 q, hd;
     };
-    __device__ static Regs load(const Row &r, uint32_t b, int s) {
+    template <class RowT>
+    __device__ static Regs load(const RowT &r, uint32_t b, int s) {
         const int c = s >> 1, h = s & 1;
         return {ld128(r, r.P[0] + 128 * b + 32 * c + 16 * h), ld128(r, r.P[1] + 16 * b)};
     }
@@ -291,7 +320,8 @@ struct Kq<MI355X_TYPE_Q5_K> {
     struct Regs {
         u32x4 q, qh, hd;
     };
-    __device__ static Regs load(const Row &r, uint32_t b, int s) {
+    template <class RowT>
+    __device__ static Regs load(const RowT &r, uint32_t b, int s) {
         const int c = s >> 1, h = s & 1;
         return {ld128(r, r.P[0] + 128 * b + 32 * c + 16 * h), ld128(r, r.P[1] + 32 * b + 16 * h),
                 ld128(r, r.P[2] + 16 * b)};
@@ -326,7 +356,8 @@ struct Kq<MI355X_TYPE_Q6_K> {
         uint32_t sw4, d;
     };
     // lane record (ql, ql, qh runs), the slice pair's scale word, d
-    __device__ static Regs load(const Row &r, uint32_t b, int s) {
+    template <class RowT>
+    __device__ static Regs load(const RowT &r, uint32_t b, int s) {
         const GPos q = gpos(r, 210, b, s);
         const u32x4 a = ld128(r, q.base + 24 * q.m);
         const u32x2 h = ld64(r, q.base + 24 * q.m + 16);
@@ -370,7 +401,8 @@ struct Kq<MI355X_TYPE_Q3_K> {
     // (sw01[kk]: the low-nibble bytes of scales kk, kk + 4, kk + 2, kk + 6;
     // sw2: scales[8..11]), d.  The loads return raw words; the exchange of h happens at decode
     // (hmask), so no load has to complete before the next one is issued.
-    __device__ static Regs load(const Row &r, uint32_t b, int s) {
+    template <class RowT>
+    __device__ static Regs load(const RowT &r, uint32_t b, int s) {
         const GPos q = gpos(r, 110, b, s);
         const u32x3 rec = ld96(r, q.base + 12 * q.m);
         const u32x3 sc = ld96(r, q.base + 96 * q.g + 12 * q.bl);
@@ -448,7 +480,8 @@ struct Kq<MI355X_TYPE_IQ4_XS> {
     __device__ static uint32_t lookup(uint32_t n) {
         return iq4_lookup(n, kT0, kT1, kT2, kT3);
     }
-    __device__ static Regs load(const Row &r, uint32_t b, int s) {
+    template <class RowT>
+    __device__ static Regs load(const RowT &r, uint32_t b, int s) {
         return {ld128(r, r.P[0] + 128 * b + 16 * s), ld64(r, r.P[1] + 8 * b)};
     }
     __device__ static float compute(const Regs &g, int s, const XSlice &x, const uint32_t *) {
@@ -482,7 +515,8 @@ struct Kq<MI355X_TYPE_IQ3_S> {
         uint32_t sg, qh, scb, d;
     };
     // lane record (qs, signs), qh byte, scale byte, d
-    __device__ static Regs load(const Row &r, uint32_t b, int s) {
+    template <class RowT>
+    __device__ static Regs load(const RowT &r, uint32_t b, int s) {
         const GPos q = gpos(r, 110, b, s);
         const u32x3 rec = ld96(r, q.base + 12 * q.m);
         return {u32x2{rec[0], rec[1]}, rec[2], ld8(r, q.base + 96 * q.g + q.m),
@@ -515,7 +549,8 @@ struct Kq<MI355X_TYPE_IQ3_XXS> {
         uint32_t aux, d;
     };
     // lane record (qs, scales_and_signs word), d
-    __device__ static Regs load(const Row &r, uint32_t b, int s) {
+    template <class RowT>
+    __device__ static Regs load(const RowT &r, uint32_t b, int s) {
         const GPos q = gpos(r, 98, b, s);
         const u32x3 rec = ld96(r, q.base + 12 * q.m);
         return {u32x2{rec[0], rec[1]}, rec[2], ld16(r, q.d)};
@@ -547,7 +582,8 @@ struct Kq<MI355X_TYPE_IQ2_S> {
         uint32_t qs, sg, qh, scb, d;
     };
     // lane record (qs, signs), the (qh, scale) byte pair, d
-    __device__ static Regs load(const Row &r, uint32_t b, int s) {
+    template <class RowT>
+    __device__ static Regs load(const RowT &r, uint32_t b, int s) {
         const GPos q = gpos(r, 82, b, s);
         const u32x2 rec = ld64(r, q.base + 8 * q.m);
         const uint32_t p = ld16(r, q.base + 64 * q.g + 2 * q.m);

@@ -300,6 +300,8 @@ int sync_iq_grids(mi355x_ctx *ctx) {
     };
     int rc = upload(g_iq3xxs_grid, &ctx->iq3xxs_grid);
     if (!rc) rc = upload(g_iq2s_grid, &ctx->iq2s_grid);
+    if (!rc && !g_iq3xxs_grid.empty()) ctx->iq3xxs_max = *std::max_element(g_iq3xxs_grid.begin(), g_iq3xxs_grid.end());
+    if (!rc && !g_iq2s_grid.empty()) ctx->iq2s_max = *std::max_element(g_iq2s_grid.begin(), g_iq2s_grid.end());
     if (!rc) ctx->grids_version = g_grid_version.load();
     return rc;
 }
@@ -417,7 +419,7 @@ void mi355x_ctx_destroy(mi355x_ctx *ctx) {
     }
     DeviceGuard dg(ctx->device);
     (void)ov_join(ctx);
-    for (void *p : {ctx->staging, ctx->xconv, ctx->mbtiles, ctx->iq3xxs_grid, ctx->iq2s_grid})
+    for (void *p : {ctx->staging, ctx->xconv, ctx->mbtiles, ctx->gemm_buf, ctx->iq3xxs_grid, ctx->iq2s_grid})
         (void)free_device(ctx, p);
     (void)stop_servers(ctx);
     (void)hipStreamSynchronize(ctx->stream);
@@ -922,6 +924,20 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
             return set_error(MI355X_EUNSUPPORTED, std::string(who) +
                                                       ": the grid is not on this context yet (one mi355x_gemv of "
                                                       "this type on the context first)");
+    }
+    // many activations: the matrix cores (every type)
+    if (ctx && M >= 2 && N > 0 && K > 0 && W && x && y && (reinterpret_cast<uintptr_t>(W) & 1) == 0 &&
+        mi355x_type_ready(type)) {
+        uint64_t total = 0;
+        int rc = check_tensor(type, N, K, &total, who);
+        if (rc) return rc;
+        DeviceGuard dg(ctx->device);
+        if (type == MI355X_TYPE_IQ3_XXS || type == MI355X_TYPE_IQ2_S) {
+            rc = sync_iq_grids(ctx);
+            if (rc) return rc;
+        }
+        GemvArgs a{type, static_cast<const uint8_t *>(W), N, K, x, false, y};
+        if (gemm_batched_supports(ctx, a, M)) return launch_gemm_batched(ctx, a, x_stride, y_stride, M, noalloc);
     }
     // Q4_0 digit-plane arithmetic: up to q4_0_mb_capacity() activations per
     // launch of the batched form (weights read once per launch)
