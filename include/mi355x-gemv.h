@@ -284,11 +284,16 @@ MI355X_API int mi355x_gemv_bf16(mi355x_ctx *ctx, int type, const void *W, int64_
 /* M activation rows at once (row m at x + m*x_stride floats, output at
  * y + m*y_stride floats); the M-row case the reference admits for weights in
  * its own buffer type and computes as M sequential GEMVs
- * (src/ggml-xdna.cpp:110-112, 287-296).  Q4_0 with the digit-plane
- * arithmetic (variants AUTO and DIGITS), rows a multiple of 256 values and
- * 16-byte aligned weights: up to 8 activations per pass over the weights
- * (one staging launch into a context buffer, one batched launch).  Other
- * cases:
+ * (src/ggml-xdna.cpp:110-112, 287-296).  In the variants AUTO and DIGITS many
+ * activations (M >= 16 for Q4_0 with an even number of blocks per row, M >= 4
+ * for the other types) run on the matrix cores, up to 512 per pass over the
+ * weights: activations as two f16 planes (22 bits), products exact, f32 sums
+ * (one launch that splits the activations into a context buffer, one product
+ * launch, and one that adds the partial sums where K is split; IQ3_XXS and
+ * IQ2_S with grids of magnitudes up to 66).  Fewer Q4_0 activations with the
+ * digit-plane arithmetic, rows a multiple of 256 values and 16-byte aligned
+ * weights: up to 8 per pass (one staging launch into a context buffer, one
+ * batched launch).  Other cases:
  * M sequential GEMVs.  Calls on one context serialise on its lock while
  * they enqueue. */
 MI355X_API int mi355x_gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,

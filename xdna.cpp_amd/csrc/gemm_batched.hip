@@ -12,26 +12,31 @@
 // 66; Q6_K and IQ4_XS need 12 bits and take a second operand with the exact
 // remainder; Q4_0 keeps its bare codes and applies the block scale to each
 // block's sum.  Activations are split into two f16 planes, hi = f16(x s) and
-// lo = f16(x s - hi) with s a power of two per (row, 256 values) that puts the
-// largest |x| in [2^14, 2^15): x s = hi + lo to 2^-22 of x, or 2^-25 absolute,
-// i.e. 2^-39 of the superblock's largest value.  Products are exact in f32 and
-// sums are f32 over 256 values (32 for Q4_0), then scaled by the superblock's
-// d and s and added in f32 over superblocks.  This is more accurate than the
-// 20- or 16-bit fixed point of the single-row kernels.
+// lo = f16(x s - hi) with s a power of two per row that puts its largest |x|
+// in [2^14, 2^15): x s = hi + lo to 2^-22 of x, or 2^-25 absolute, i.e. 2^-39
+// of the row's largest value.  Products are exact in f32 and sums are f32 over
+// 256 values (32 for Q4_0), scaled by the superblock's d and added in f32 over
+// superblocks.  This is more accurate than the 20- or 16-bit fixed point of
+// the single-row kernels.
 //
 // Work split.  A workgroup of 4 wavefronts computes 256 output columns (weight
 // rows) x 32 or 64 activation rows; a wavefront 64 columns as two 32-wide
 // MFMA tiles, so that each activation operand read from LDS feeds two
-// products.  K is walked in half superblocks: the activation planes of the
-// next half travel to LDS directly (buffer_load ... lds) and the next half's
-// weights to registers while this half is multiplied.  Where the tiles leave
-// CUs idle the superblocks are split over gridDim.y segments whose f32
-// partials a second kernel adds in segment order.
+// products.  K is walked in half superblocks of 8 operand steps: the
+// activation planes of the next half travel to LDS directly (global_load_lds)
+// and its weights to registers while this half is multiplied, and each step's
+// operands are decoded dword by dword between the products of the step before
+// (a sched_barrier after every product keeps that order: left alone, the
+// compiler decodes a whole half first).  Where the tiles leave CUs idle the
+// superblocks are split over gridDim.y segments whose f32 partials a second
+// kernel adds in segment order.
 //
-// Measured on MI355X, us per call (sequential or 8-row passes before): Q4_0
-// 17408x5120 M = 512 395 (2700), Q6_K 4096x14336 M = 512 232 (6330), Q4_K
-// 14336x4096 M = 37 40 (256); 231-259 TFLOP/s of useful products, each two
-// MFMAs (three for Q6_K).
+// What bounds it.  MFMAs on real data take 19 ns each here (power; 13 ns at
+// full clock); with the decode between them 21 ns, and two (Q6_K, IQ4_XS:
+// three) make one useful product.  On top of that come the weights' loads,
+// where the 64 lanes of a load touch 64 rows.  us per call on MI355X
+// (sequential or 8-row passes before): Q4_0 17408x5120 M = 512 301 (2710),
+// Q6_K 4096x14336 M = 512 218 (6310), Q4_K 14336x4096 M = 37 37 (252).
 #include "internal.h"
 #include "kq_device.h"
 #include "q4_0_layout.h"
@@ -39,6 +44,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 
 namespace mi355x {
 namespace {
@@ -67,7 +73,7 @@ struct GemmArgs {
     int nseg;
     const uint8_t *planes;  // [superblock][half][Mp][512]
     const _Float16 *sums;   // [superblock][Mp][16]
-    const float *unit;      // [superblock][Mp]
+    const float *unit;      // [Mp]: 1 / s of each row
     const float *x;         // CONV: the activations themselves
     int64_t x_stride;
     int x_al16;
@@ -114,43 +120,44 @@ __device__ __forceinline__ float wave_max(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// Four values of a row (`left` of the superblock's 256 exist).
+__device__ __forceinline__ float4 load_x4(const float *x, int i0, int left, bool al16) {
+    if (al16 && i0 + 3 < left) return *reinterpret_cast<const float4 *>(x + i0);
+    float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i0 < left) f.x = x[i0];
+    if (i0 + 1 < left) f.y = x[i0 + 1];
+    if (i0 + 2 < left) f.z = x[i0 + 2];
+    if (i0 + 3 < left) f.w = x[i0 + 3];
+    return f;
+}
+__device__ __forceinline__ float abs_max4(const float4 &f) {
+    return fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w)));
+}
+
+// Scale of a row whose largest |x| is mx: s = 2^(14 - E) for mx in
+// [2^E, 2^(E+1)), E >= -110 (smaller and all-zero rows take 2^124), and 1 / s.
+__device__ __forceinline__ float row_scale(float mx, float &unit) {
+    const int e = min(max(static_cast<int>(__builtin_bit_cast(uint32_t, mx) >> 23), 17), 254);  // biased E
+    unit = __builtin_bit_cast(float, static_cast<uint32_t>(e - 14) << 23);
+    return __builtin_bit_cast(float, static_cast<uint32_t>(268 - e) << 23);
+}
+
 struct XPlanes {
-    uint2 hi, lo;  // this lane's 4 values of each plane, in run order
-    float unit;    // 1 / s
+    uint2 hi, lo;         // this lane's 4 values of each plane, in run order
     _Float16 s_hi, s_lo;  // lanes 8j: sum of sub-block j (times s / 32)
 };
 
 // One superblock of one activation row by a whole wavefront: lane l converts
-// values 4l .. 4l + 3 (`left` of the 256 exist, the rest are zero).
-__device__ __forceinline__ XPlanes convert_superblock(const float *x, int left, bool al16, int lane) {
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
-    const int i0 = 4 * lane;
-    if (al16 && i0 + 3 < left) {
-        const float4 f = *reinterpret_cast<const float4 *>(x + i0);
-        v[0] = f.x;
-        v[1] = f.y;
-        v[2] = f.z;
-        v[3] = f.w;
-    } else {
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            if (i0 + t < left) v[t] = x[i0 + t];
-    }
-    const float mx = wave_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
-    // s = 2^(14 - E) for max in [2^E, 2^(E+1)), E >= -110 (an all-zero or
-    // smaller superblock takes 2^124)
-    const int e = max(static_cast<int>(__builtin_bit_cast(uint32_t, mx) >> 23), 17);  // biased E
-    const float s = __builtin_bit_cast(float, static_cast<uint32_t>(268 - min(e, 254)) << 23);
-    XPlanes r;
-    r.unit = __builtin_bit_cast(float, static_cast<uint32_t>(min(e, 254) - 14) << 23);
-    float w[4];
+// values 4l .. 4l + 3.
+__device__ __forceinline__ XPlanes convert_superblock(const float4 &f, float s) {
+    const float w[4] = {f.x * s, f.y * s, f.z * s, f.w * s};
     _Float16 h[4], l[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        w[t] = v[t] * s;
         h[t] = static_cast<_Float16>(w[t]);
         l[t] = static_cast<_Float16>(w[t] - static_cast<float>(h[t]));
     }
+    XPlanes r;
     r.hi = make_uint2(u2(f16x2{h[0], h[2]}), u2(f16x2{h[1], h[3]}));
     r.lo = make_uint2(u2(f16x2{l[0], l[2]}), u2(f16x2{l[1], l[3]}));
     float sum = (w[0] + w[1]) + (w[2] + w[3]);
@@ -178,30 +185,59 @@ __device__ __forceinline__ void store_superblock(const XPlanes &c, int m, int la
     }
 }
 
-// Planes, sums and units of M activation rows: one wavefront per (row,
-// superblock).
-__global__ __launch_bounds__(256) void gemm_planes_kernel(const float *x, int64_t x_stride, int64_t K, int x_al16,
-                                                          int M, int Mp, int B, uint8_t *planes, _Float16 *sums,
-                                                          float *unit) {
-    const int lane = threadIdx.x & 63;
-    const int64_t task = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (task >= static_cast<int64_t>(M) * B) return;
-    const int m = static_cast<int>(task / B), b = static_cast<int>(task % B);
-    const int64_t left = K - 256 * static_cast<int64_t>(b);
-    const XPlanes c = convert_superblock(x + m * x_stride + 256 * static_cast<int64_t>(b),
-                                         static_cast<int>(left < 256 ? left : 256), x_al16 != 0, lane);
-    uint8_t *h0 = planes + (static_cast<int64_t>(2 * b) * Mp + m) * kGmHalfBytes;
-    store_superblock(c, m, lane, h0, h0 + static_cast<int64_t>(Mp) * kGmHalfBytes,
-                     sums + (static_cast<int64_t>(b) * Mp + m) * 16);
-    if (lane == 0) unit[static_cast<int64_t>(b) * Mp + m] = c.unit;
+// Planes, sums and units of the activation rows: one workgroup per row, its
+// wavefronts taking the superblocks in turn; the first kPlKeep of each stay in
+// registers between the row's maximum and the conversion.
+constexpr int kPlThreads = 1024, kPlWavesG = kPlThreads / 64, kPlKeep = 4;
+__global__ __launch_bounds__(kPlThreads) void gemm_planes_kernel(const float *x, int64_t x_stride, int64_t K,
+                                                                 int x_al16, int Mp, int B, uint8_t *planes,
+                                                                 _Float16 *sums, float *unit) {
+    __shared__ float smax[kPlWavesG];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m = blockIdx.x;
+    const float *xr = x + m * x_stride;
+    auto load = [&](int b) {
+        const int64_t left = K - 256 * static_cast<int64_t>(b);
+        return load_x4(xr + 256 * static_cast<int64_t>(b), 4 * lane, static_cast<int>(left < 256 ? left : 256), x_al16 != 0);
+    };
+    float4 keep[kPlKeep];
+    float mx = 0.f;
+#pragma unroll
+    for (int k = 0; k < kPlKeep; ++k) {
+        const int b = wave + kPlWavesG * k;
+        keep[k] = b < B ? load(b) : make_float4(0.f, 0.f, 0.f, 0.f);
+        mx = fmaxf(mx, abs_max4(keep[k]));
+    }
+    for (int b = wave + kPlWavesG * kPlKeep; b < B; b += kPlWavesG) mx = fmaxf(mx, abs_max4(load(b)));
+    mx = wave_max(mx);
+    if (lane == 0) smax[wave] = mx;
+    __syncthreads();
+    mx = wave_max(smax[lane & (kPlWavesG - 1)]);
+    float u;
+    const float s = row_scale(mx, u);
+    if (threadIdx.x == 0) unit[m] = u;
+    auto put = [&](int b, const float4 &f) {
+        uint8_t *h0 = planes + (static_cast<int64_t>(2 * b) * Mp + m) * kGmHalfBytes;
+        store_superblock(convert_superblock(f, s), m, lane, h0, h0 + static_cast<int64_t>(Mp) * kGmHalfBytes,
+                         sums + (static_cast<int64_t>(b) * Mp + m) * 16);
+    };
+#pragma unroll
+    for (int k = 0; k < kPlKeep; ++k) {
+        const int b = wave + kPlWavesG * k;
+        if (b < B) put(b, keep[k]);
+    }
+    for (int b = wave + kPlWavesG * kPlKeep; b < B; b += kPlWavesG) put(b, load(b));
 }
 
 // ---- weight decode --------------------------------------------------------------
 // Gw<TYPE>: the weights of one lane (one weight row) for slice s of a
 // superblock as four f16 operands, operand p the run at position p of the
-// slice (run_of).  decode's `half` and `q` are compile-time constants at every
-// call (s = 4 half + 2 q + h, h = lane / 32).  kWide types leave the exact
-// remainder of codes times scales in lo; d(regs) is the superblock's scale.
+// slice (run_of).  dword(p, j) gives dword j of operand p: the run's values
+// (0, 2), (1, 3), (4, 6), (5, 7); kWide types leave the exact remainder of
+// code times scale in lo.  half, q, p and j are compile-time constants at
+// every call (s = 4 half + 2 q + h, h = lane / 32); what the dwords share
+// (scales) is written into each and kept by the compiler.  Codebook types
+// read their kLooks table entries of operand p ahead of time (look).  d(regs)
+// is the superblock's scale.
 template <int TYPE>
 struct Gw;
 
@@ -211,49 +247,36 @@ __device__ __forceinline__ uint32_t scale_pair_k4(int c, const u32x4 &hd) {
     const uint32_t a2 = hd[1] >> sh, c2 = hd[3] >> sh;
     return c < 2 ? (a2 & 0x3F3Fu) : ((c2 & 0x0F0Fu) | ((a2 >> 2) & 0x3030u));
 }
-// byte B of w as an f16 integer in both halves
-template <int B>
+// byte B of w less BIAS as f16 in both halves
+template <int B, int BIAS = 0>
 __device__ __forceinline__ f16x2 byte_h2(uint32_t w) {
-    return h2(__builtin_amdgcn_perm(w, w, 0x0C000C00u | (static_cast<uint32_t>(B) << 16) | B) | kH1024) - h2s(1024.f);
-}
-// the same less BIAS
-template <int B, int BIAS>
-__device__ __forceinline__ f16x2 byte_h2_biased(uint32_t w) {
     return h2(__builtin_amdgcn_perm(w, w, 0x0C000C00u | (static_cast<uint32_t>(B) << 16) | B) | kH1024) -
            h2s(1024.f + BIAS);
 }
 
+// Q4_K, Q5_K: operands 0, 1 the low nibbles of code bytes 0-7, 8-15, operands
+// 2, 3 the high nibbles.  The high codes stay in place (16 times the code) and
+// the fma that removes the 1024 also applies the scale: sc <= 63, so every
+// product and sum is exact.
 template <bool Q5, class Regs>
-__device__ __forceinline__ void k45_decode(const Regs &g, int half, int q, f16x8 (&hi)[4]) {
-    const int c = 2 * half + q;
+__device__ __forceinline__ uint32_t k45_dword(const Regs &g, int half, int q, int p, int j) {
+    const int c = 2 * half + q, i = 2 * (p & 1) + (j >> 1);
     const uint32_t sp = scale_pair_k4(c, g.hd);
-    const f16x2 sc0 = byte_h2<0>(sp), sc1 = byte_h2<1>(sp) * h2s(0.0625f);
-    const f16x2 o0 = sc0 * h2s(-1024.f), o1 = sc1 * h2s(-1024.f);  // exact: sc <= 63
-    uint32_t lo[8], up[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t w = g.q[i], w8 = w >> 8;
-        uint32_t a = (w & 0x000F000Fu) | kH1024, b = (w8 & 0x000F000Fu) | kH1024;
-        uint32_t e = (w & 0x00F000F0u) | kH1024, f = (w8 & 0x00F000F0u) | kH1024;
-        if constexpr (Q5) {
-            // high bit 2c of each qh byte to bit 4 of the low codes, bit
-            // 2c + 1 to bit 8 of the in-place high codes
-            const uint32_t qh = g.qh[i];
+    const f16x2 sc = p < 2 ? byte_h2<0>(sp) : byte_h2<1>(sp) * h2s(0.0625f);
+    const uint32_t w = (j & 1) ? g.q[i] >> 8 : g.q[i];
+    uint32_t a = (w & (p < 2 ? 0x000F000Fu : 0x00F000F0u)) | kH1024;
+    if constexpr (Q5) {
+        // high bit 2c of each qh byte to bit 4 of the low codes, bit 2c + 1
+        // to bit 8 of the in-place high codes
+        const uint32_t qh = g.qh[i];
+        if (p < 2) {
             const uint32_t t = 2 * c <= 4 ? qh << (4 - 2 * c) : qh >> (2 * c - 4);
-            a |= t & 0x00100010u;
-            b |= (t >> 8) & 0x00100010u;
-            e |= (7 - 2 * c >= 0 ? qh << (7 - 2 * c) : qh) & 0x01000100u;
-            f |= (qh >> (2 * c + 1)) & 0x01000100u;
+            a |= ((j & 1) ? t >> 8 : t) & 0x00100010u;
+        } else {
+            a |= ((j & 1) ? qh >> (2 * c + 1) : qh << (7 - 2 * c)) & 0x01000100u;
         }
-        lo[2 * i] = u2(pk_fma(h2(a), sc0, o0));
-        lo[2 * i + 1] = u2(pk_fma(h2(b), sc0, o0));
-        up[2 * i] = u2(pk_fma(h2(e), sc1, o1));
-        up[2 * i + 1] = u2(pk_fma(h2(f), sc1, o1));
     }
-    hi[0] = frag8(lo[0], lo[1], lo[2], lo[3]);
-    hi[1] = frag8(lo[4], lo[5], lo[6], lo[7]);
-    hi[2] = frag8(up[0], up[1], up[2], up[3]);
-    hi[3] = frag8(up[4], up[5], up[6], up[7]);
+    return u2(pk_fma(h2(a), sc, sc * h2s(-1024.f)));
 }
 // the 8 sub-block mins of a superblock in run order
 __device__ __forceinline__ f16x8 k4_mins(const u32x4 &hd) {
@@ -267,21 +290,23 @@ __device__ __forceinline__ f16x8 k4_mins(const u32x4 &hd) {
 template <>
 struct Gw<MI355X_TYPE_Q4_K> {
     static constexpr bool kWide = false, kMins = true;
+    static constexpr int kLooks = 0;
     using Regs = Kq<MI355X_TYPE_Q4_K>::Regs;
     __device__ static Regs load(const LaneRow &r, uint32_t b, int s) { return Kq<MI355X_TYPE_Q4_K>::load(r, b, s); }
     __device__ static float d(const Regs &g) { return half_f(g.hd[0] & 0xFFFF); }
-    __device__ static void decode(const Regs &g, int half, int q, const uint2 *, f16x8 (&hi)[4], f16x8 (&)[4]) {
-        k45_decode<false>(g, half, q, hi);
+    __device__ static void dword(const Regs &g, int half, int q, int p, int j, const uint2 *, uint32_t &hi, uint32_t &) {
+        hi = k45_dword<false>(g, half, q, p, j);
     }
 };
 template <>
 struct Gw<MI355X_TYPE_Q5_K> {
     static constexpr bool kWide = false, kMins = true;
+    static constexpr int kLooks = 0;
     using Regs = Kq<MI355X_TYPE_Q5_K>::Regs;
     __device__ static Regs load(const LaneRow &r, uint32_t b, int s) { return Kq<MI355X_TYPE_Q5_K>::load(r, b, s); }
     __device__ static float d(const Regs &g) { return half_f(g.hd[0] & 0xFFFF); }
-    __device__ static void decode(const Regs &g, int half, int q, const uint2 *, f16x8 (&hi)[4], f16x8 (&)[4]) {
-        k45_decode<true>(g, half, q, hi);
+    __device__ static void dword(const Regs &g, int half, int q, int p, int j, const uint2 *, uint32_t &hi, uint32_t &) {
+        hi = k45_dword<true>(g, half, q, p, j);
     }
 };
 
@@ -291,45 +316,34 @@ __device__ __forceinline__ void wide_mul(f16x2 v, f16x2 sc, uint32_t &hi, uint32
     hi = u2(p);
     lo = u2(pk_fma(v, sc, -p));
 }
+// w << sh for sh >= 0, else w >> -sh
+__device__ __forceinline__ uint32_t shift(uint32_t w, int sh) { return sh >= 0 ? w << sh : w >> -sh; }
 
 template <>
 struct Gw<MI355X_TYPE_Q6_K> {
     static constexpr bool kWide = true, kMins = false;
+    static constexpr int kLooks = 0;
     using Regs = Kq<MI355X_TYPE_Q6_K>::Regs;
     __device__ static Regs load(const LaneRow &r, uint32_t b, int s) { return Kq<MI355X_TYPE_Q6_K>::load(r, b, s); }
     __device__ static float d(const Regs &g) { return half_f(g.d); }
-    __device__ static void decode(const Regs &g, int, int, const uint2 *, f16x8 (&hi)[4], f16x8 (&lo)[4]) {
-        uint32_t H[4][4], L[4][4];
+    __device__ static void dword(const Regs &g, int, int, int p, int j, const uint2 *, uint32_t &hi, uint32_t &lo) {
         const uint32_t sw = g.sw4 ^ 0x80808080u;  // int8 scales + 128
-        const f16x2 sc[4] = {byte_h2_biased<0, 128>(sw), byte_h2_biased<1, 128>(sw), byte_h2_biased<2, 128>(sw),
-                             byte_h2_biased<3, 128>(sw)};
-        const f16x2 off = h2s(1024.f + 32.f);
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-            const uint32_t A = g.qa[w], Bq = g.qb[w], Q = g.qh[w];
-            const uint32_t code[4][2] = {
-                {(A & 0x000F000Fu) | ((Q << 4) & 0x00300030u), ((A >> 8) & 0x000F000Fu) | ((Q >> 4) & 0x00300030u)},
-                {(Bq & 0x000F000Fu) | ((Q << 2) & 0x00300030u), ((Bq >> 8) & 0x000F000Fu) | ((Q >> 6) & 0x00300030u)},
-                {((A >> 4) & 0x000F000Fu) | (Q & 0x00300030u), ((A >> 12) & 0x000F000Fu) | ((Q >> 8) & 0x00300030u)},
-                {((Bq >> 4) & 0x000F000Fu) | ((Q >> 2) & 0x00300030u),
-                 ((Bq >> 12) & 0x000F000Fu) | ((Q >> 10) & 0x00300030u)}};
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-                    wide_mul(h2(code[j][t] | kH1024) - off, sc[j], H[j][2 * w + t], L[j][2 * w + t]);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            hi[j] = frag8(H[j][0], H[j][1], H[j][2], H[j][3]);
-            lo[j] = frag8(L[j][0], L[j][1], L[j][2], L[j][3]);
-        }
+        const f16x2 sc = p == 0   ? byte_h2<0, 128>(sw)
+                         : p == 1 ? byte_h2<1, 128>(sw)
+                         : p == 2 ? byte_h2<2, 128>(sw)
+                                  : byte_h2<3, 128>(sw);
+        // nibble p / 2 of the first (p even) or second ql run, bits 2p of qh above it
+        const int w = j >> 1, o = 8 * (j & 1);
+        const uint32_t A = (p & 1) ? g.qb[w] : g.qa[w];
+        const uint32_t c = ((A >> (4 * (p >> 1) + o)) & 0x000F000Fu) | (shift(g.qh[w], 4 - 2 * p - o) & 0x00300030u);
+        wide_mul(h2(c | kH1024) - h2s(1024.f + 32.f), sc, hi, lo);
     }
 };
 
 template <>
 struct Gw<MI355X_TYPE_Q3_K> {
     static constexpr bool kWide = false, kMins = false;
+    static constexpr int kLooks = 0;
     // as Kq<Q3_K>::Regs with both halves of the slice's 8 hmask bytes
     struct Regs {
         u32x2 q, hm, sw01;
@@ -345,141 +359,100 @@ struct Gw<MI355X_TYPE_Q3_K> {
         return {q, u32x2{h0, h1}, u32x2{sc[0], sc[1]}, sc[2], ld16(r, p.d)};
     }
     __device__ static float d(const Regs &g) { return half_f(g.d); }
-    __device__ static void decode(const Regs &g, int half, int q, const uint2 *, f16x8 (&hi)[4], f16x8 (&)[4]) {
+    __device__ static void dword(const Regs &g, int half, int q, int p, int j, const uint2 *, uint32_t &hi, uint32_t &) {
         // the four 6-bit scales in one word, bytes in run order 0, 2, 1, 3
         // (KqDg<Q3_K>); kk = q, hh = half
         const uint32_t Lw = q ? g.sw01[1] : g.sw01[0];
         const uint32_t Hw = g.sw2 >> (8 * q + 4 * half);
         const uint32_t SC = ((Lw >> (4 * half)) & 0x0F0F0F0Fu) | ((Hw & 0x00030003u) << 4) | ((Hw & 0x000C000Cu) << 10);
-        const f16x2 sc[4] = {byte_h2_biased<0, 32>(SC), byte_h2_biased<2, 32>(SC), byte_h2_biased<1, 32>(SC),
-                             byte_h2_biased<3, 32>(SC)};
-        uint32_t H[4][4];
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                // code bits in place (4^j times the code), the hmask bit above
-                const uint32_t m2 = 0x00030003u << (2 * j), mh = 0x00040004u << (2 * j);
-                const int sh = j + 2 - 4 * half;  // hmask bit 4 half + j to bit 2j + 2
-                const uint32_t h0 = sh >= 0 ? g.hm[w] << sh : g.hm[w] >> -sh;
-                const uint32_t h1 = 8 - sh >= 0 ? g.hm[w] >> (8 - sh) : g.hm[w];
-                const uint32_t a = (g.q[w] & m2) | (h0 & mh) | kH1024;
-                const uint32_t b = ((g.q[w] >> 8) & m2) | (h1 & mh) | kH1024;
-                const float f = static_cast<float>(1 << (2 * j));
-                const f16x2 o = h2s(1024.f + 4.f * f), sj = sc[j] * h2s(1.f / f);
-                H[j][2 * w] = u2((h2(a) - o) * sj);
-                H[j][2 * w + 1] = u2((h2(b) - o) * sj);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) hi[j] = frag8(H[j][0], H[j][1], H[j][2], H[j][3]);
+        const f16x2 sc = p == 0   ? byte_h2<0, 32>(SC)
+                         : p == 1 ? byte_h2<2, 32>(SC)
+                         : p == 2 ? byte_h2<1, 32>(SC)
+                                  : byte_h2<3, 32>(SC);
+        // code bits in place (4^p times the code), the hmask bit above them:
+        // bit 4 half + p of the byte to bit 2p + 2
+        const int w = j >> 1, o = 8 * (j & 1);
+        const uint32_t m2 = 0x00030003u << (2 * p), mh = 0x00040004u << (2 * p);
+        const float f = static_cast<float>(1 << (2 * p));
+        const uint32_t a = ((g.q[w] >> o) & m2) | (shift(g.hm[w], p + 2 - 4 * half - o) & mh) | kH1024;
+        hi = u2((h2(a) - h2s(1024.f + 4.f * f)) * (sc * h2s(1.f / f)));
     }
 };
 
 template <>
 struct Gw<MI355X_TYPE_IQ4_XS> {
     static constexpr bool kWide = true, kMins = false;
+    static constexpr int kLooks = 0;
     using Regs = Kq<MI355X_TYPE_IQ4_XS>::Regs;
     __device__ static Regs load(const LaneRow &r, uint32_t b, int s) { return Kq<MI355X_TYPE_IQ4_XS>::load(r, b, s); }
     __device__ static float d(const Regs &g) { return half_f(g.hd[0] & 0xFFFF); }
-    __device__ static void decode(const Regs &g, int half, int q, const uint2 *, f16x8 (&hi)[4], f16x8 (&lo)[4]) {
+    __device__ static void dword(const Regs &g, int half, int q, int p, int j, const uint2 *, uint32_t &hi, uint32_t &lo) {
         const uint32_t s = static_cast<uint32_t>(4 * half + 2 * q) + (__lane_id() >> 5);
         const uint32_t sh = g.hd[0] >> 16;
         const uint32_t ls = ((g.hd[1] >> (4 * s)) & 15u) | (((sh >> (2 * s)) & 3u) << 4);
-        const f16x2 sc = byte_h2_biased<0, 32>(ls);
-        const f16x2 off = h2s(1024.f + 128.f);  // the codebook bytes are kvalues + 128
-        uint32_t H[16], L[16];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t a = Kq<MI355X_TYPE_IQ4_XS>::lookup(g.q[i] & 0x0F0F0F0Fu);
-            const uint32_t b = Kq<MI355X_TYPE_IQ4_XS>::lookup((g.q[i] >> 4) & 0x0F0F0F0Fu);
-            wide_mul(h2((a & 0x00FF00FFu) | kH1024) - off, sc, H[2 * i], L[2 * i]);
-            wide_mul(h2(((a >> 8) & 0x00FF00FFu) | kH1024) - off, sc, H[2 * i + 1], L[2 * i + 1]);
-            wide_mul(h2((b & 0x00FF00FFu) | kH1024) - off, sc, H[8 + 2 * i], L[8 + 2 * i]);
-            wide_mul(h2(((b >> 8) & 0x00FF00FFu) | kH1024) - off, sc, H[9 + 2 * i], L[9 + 2 * i]);
-        }
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            hi[p] = frag8(H[4 * p], H[4 * p + 1], H[4 * p + 2], H[4 * p + 3]);
-            lo[p] = frag8(L[4 * p], L[4 * p + 1], L[4 * p + 2], L[4 * p + 3]);
-        }
+        const uint32_t w = g.q[2 * (p & 1) + (j >> 1)];
+        const uint32_t a = Kq<MI355X_TYPE_IQ4_XS>::lookup((p < 2 ? w : w >> 4) & 0x0F0F0F0Fu);
+        // the codebook bytes are kvalues + 128
+        wide_mul(h2((((j & 1) ? a >> 8 : a) & 0x00FF00FFu) | kH1024) - h2s(1024.f + 128.f), byte_h2<0, 32>(ls), hi, lo);
     }
 };
 
-// Sign masks of the f16 pairs of 8 values from their sign byte: pairs (0, 2),
-// (1, 3), (4, 6), (5, 7) of the byte's bits.
-struct SignMasks {
-    uint32_t m[4];
-};
-__device__ __forceinline__ SignMasks sign_masks(uint32_t b) {
-    const uint32_t t = b | (b << 14);  // bit i also at 14 + i: bits 2i and 16 + .. meet in a halfword pair
-    return {{(t << 15) & 0x80008000u, (t << 14) & 0x80008000u, (t << 11) & 0x80008000u, (t << 10) & 0x80008000u}};
-}
-// 8 grid magnitudes (two f16 table entries of 4) with signs, times sc
-__device__ __forceinline__ f16x8 signed_run(uint2 e0, uint2 e1, uint32_t signs, f16x2 sc) {
-    const SignMasks s = sign_masks(signs);
-    return frag8(u2(h2(e0.x ^ s.m[0]) * sc), u2(h2(e0.y ^ s.m[1]) * sc), u2(h2(e1.x ^ s.m[2]) * sc),
-                 u2(h2(e1.y ^ s.m[3]) * sc));
+// Dword j of 8 grid magnitudes with the signs of byte `signs`, times sc: m the
+// f16 pair of values (0, 2), (1, 3), (4, 6) or (5, 7); bit i of the byte and
+// its copy at 14 + i meet in the sign bits of one pair.
+__device__ __forceinline__ uint32_t signed_dword(uint32_t m, uint32_t signs, int j, f16x2 sc) {
+    const uint32_t t = signs | (signs << 14);
+    return u2(h2(m ^ ((t << (j < 2 ? 15 - j : 13 - j)) & 0x80008000u)) * sc);
 }
 
 template <>
 struct Gw<MI355X_TYPE_IQ3_S> {
     static constexpr bool kWide = false, kMins = false;
+    static constexpr int kLooks = 2;
     using Regs = Kq<MI355X_TYPE_IQ3_S>::Regs;
     __device__ static Regs load(const LaneRow &r, uint32_t b, int s) { return Kq<MI355X_TYPE_IQ3_S>::load(r, b, s); }
     __device__ static float d(const Regs &g) { return half_f(g.d); }
-    __device__ static void decode(const Regs &g, int, int, const uint2 *tab, f16x8 (&hi)[4], f16x8 (&)[4]) {
+    __device__ static uint2 look(const Regs &g, int p, int k, const uint2 *tab) {
+        return tab[byte_u(g.qs[p >> 1], 2 * (p & 1) + k) | (((g.qh >> (2 * p + k)) & 1u) << 8)];
+    }
+    __device__ static void dword(const Regs &g, int, int, int p, int j, const uint2 *e, uint32_t &hi, uint32_t &) {
         const uint32_t n = (g.scb >> ((__lane_id() >> 5) * 4)) & 15u;
-        const f16x2 sc = byte_h2<0>(2 * n + 1);
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const uint32_t w = g.qs[p >> 1];
-            const uint32_t i0 = byte_u(w, 2 * (p & 1)) | (((g.qh >> (2 * p)) & 1u) << 8);
-            const uint32_t i1 = byte_u(w, 2 * (p & 1) + 1) | (((g.qh >> (2 * p + 1)) & 1u) << 8);
-            hi[p] = signed_run(tab[i0], tab[i1], byte_u(g.sg, p), sc);
-        }
+        hi = signed_dword((j & 1) ? e[j >> 1].y : e[j >> 1].x, byte_u(g.sg, p), j, byte_h2<0>(2 * n + 1));
     }
 };
 
 template <>
 struct Gw<MI355X_TYPE_IQ3_XXS> {
     static constexpr bool kWide = false, kMins = false;
+    static constexpr int kLooks = 2;
     using Regs = Kq<MI355X_TYPE_IQ3_XXS>::Regs;
     __device__ static Regs load(const LaneRow &r, uint32_t b, int s) { return Kq<MI355X_TYPE_IQ3_XXS>::load(r, b, s); }
     // (0.5 + n) / 2 = (2 n + 1) / 4
     __device__ static float d(const Regs &g) { return 0.25f * half_f(g.d); }
-    __device__ static void decode(const Regs &g, int, int, const uint2 *tab, f16x8 (&hi)[4], f16x8 (&)[4]) {
-        const f16x2 sc = byte_h2<0>(2 * (g.aux >> 28) + 1);
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const uint32_t w = g.qs[p >> 1];
-            hi[p] = signed_run(tab[byte_u(w, 2 * (p & 1))], tab[byte_u(w, 2 * (p & 1) + 1)],
-                               ksigns((g.aux >> (7 * p)) & 127u), sc);
-        }
+    __device__ static uint2 look(const Regs &g, int p, int k, const uint2 *tab) {
+        return tab[byte_u(g.qs[p >> 1], 2 * (p & 1) + k)];
+    }
+    __device__ static void dword(const Regs &g, int, int, int p, int j, const uint2 *e, uint32_t &hi, uint32_t &) {
+        hi = signed_dword((j & 1) ? e[j >> 1].y : e[j >> 1].x, ksigns((g.aux >> (7 * p)) & 127u), j,
+                          byte_h2<0>(2 * (g.aux >> 28) + 1));
     }
 };
 
 template <>
 struct Gw<MI355X_TYPE_IQ2_S> {
     static constexpr bool kWide = false, kMins = false;
+    static constexpr int kLooks = 1;  // 8 magnitudes as bytes (f16 entries would take 16 KB and a workgroup of the CU)
     using Regs = Kq<MI355X_TYPE_IQ2_S>::Regs;
     __device__ static Regs load(const LaneRow &r, uint32_t b, int s) { return Kq<MI355X_TYPE_IQ2_S>::load(r, b, s); }
     // (0.5 + n) / 4 = (2 n + 1) / 8
     __device__ static float d(const Regs &g) { return 0.125f * half_f(g.d); }
-    __device__ static void decode(const Regs &g, int, int, const uint2 *tab, f16x8 (&hi)[4], f16x8 (&)[4]) {
-        // the table keeps the grid's bytes: an f16 table would take 16 KB and
-        // the second workgroup of a CU
-        const f16x2 sc[2] = {byte_h2<0>(2 * (g.scb & 15u) + 1), byte_h2<0>(2 * (g.scb >> 4) + 1)};
-        const f16x2 k = h2s(1024.f);
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const uint2 e = tab[byte_u(g.qs, p) | (((g.qh >> (2 * p)) & 3u) << 8)];
-            const uint2 e0 = make_uint2(u2(h2((e.x & 0x00FF00FFu) | kH1024) - k),
-                                        u2(h2(((e.x >> 8) & 0x00FF00FFu) | kH1024) - k));
-            const uint2 e1 = make_uint2(u2(h2((e.y & 0x00FF00FFu) | kH1024) - k),
-                                        u2(h2(((e.y >> 8) & 0x00FF00FFu) | kH1024) - k));
-            hi[p] = signed_run(e0, e1, byte_u(g.sg, p), sc[p >> 1]);
-        }
+    __device__ static uint2 look(const Regs &g, int p, int, const uint2 *tab) {
+        return tab[byte_u(g.qs, p) | (((g.qh >> (2 * p)) & 3u) << 8)];
+    }
+    __device__ static void dword(const Regs &g, int, int, int p, int j, const uint2 *e, uint32_t &hi, uint32_t &) {
+        const uint32_t b = j < 2 ? e[0].x : e[0].y;
+        const uint32_t m = u2(h2((((j & 1) ? b >> 8 : b) & 0x00FF00FFu) | kH1024) - h2s(1024.f));
+        hi = signed_dword(m, byte_u(g.sg, p), j, byte_h2<0>(2 * (p < 2 ? g.scb & 15u : g.scb >> 4) + 1));
     }
 };
 
@@ -491,32 +464,23 @@ struct Q40Regs {
     u32x4 q;
     uint32_t d[2];  // fp16 of blocks 2q, 2q + 1
 };
-__device__ __forceinline__ void q40_decode(const Q40Regs &g, f16x8 (&w)[2][2]) {
-    const auto s0 = __builtin_amdgcn_permlane32_swap(g.q[0], g.q[2], false, false);
-    const auto s1 = __builtin_amdgcn_permlane32_swap(g.q[1], g.q[3], false, false);
-    const uint32_t v[2][2] = {{static_cast<uint32_t>(s0[0]), static_cast<uint32_t>(s1[0])},
-                              {static_cast<uint32_t>(s0[1]), static_cast<uint32_t>(s1[1])}};
-    const f16x2 o0 = h2s(-1032.f), o1 = h2s(-72.f), c = h2s(0.0625f);
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        uint32_t L[4], U[4];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            // resident nibbles are q - 8 in two's complement: flip the sign bit
-            const uint32_t a = v[e][i], b = a >> 8;
-            L[2 * i] = u2(h2((a & 0x000F000Fu) ^ 0x64086408u) + o0);
-            L[2 * i + 1] = u2(h2((b & 0x000F000Fu) ^ 0x64086408u) + o0);
-            U[2 * i] = u2(pk_fma(h2((a & 0x00F000F0u) ^ 0x64806480u), c, o1));
-            U[2 * i + 1] = u2(pk_fma(h2((b & 0x00F000F0u) ^ 0x64806480u), c, o1));
-        }
-        w[e][0] = frag8(L[0], L[1], L[2], L[3]);
-        w[e][1] = frag8(U[0], U[1], U[2], U[3]);
-    }
+// dword j of operand i (0: low nibbles, 1: high) of block e
+__device__ __forceinline__ uint32_t q40_dword(const Q40Regs &g, int e, int i, int j) {
+    const auto sw = j < 2 ? __builtin_amdgcn_permlane32_swap(g.q[0], g.q[2], false, false)
+                          : __builtin_amdgcn_permlane32_swap(g.q[1], g.q[3], false, false);
+    const uint32_t v = static_cast<uint32_t>(sw[e]);
+    const uint32_t a = (j & 1) ? v >> 8 : v;
+    // resident nibbles are q - 8 in two's complement: flip the sign bit
+    return i == 0 ? u2(h2((a & 0x000F000Fu) ^ 0x64086408u) + h2s(-1032.f))
+                  : u2(pk_fma(h2((a & 0x00F000F0u) ^ 0x64806480u), h2s(0.0625f), h2s(-72.f)));
 }
 
-// LDS words of the codebook table
+// entries of the LDS codebook table
 constexpr int gm_table_entries(int type) {
-    return type == MI355X_TYPE_IQ3_S ? kIq3sGridSize : type == MI355X_TYPE_IQ3_XXS ? 256 : type == MI355X_TYPE_IQ2_S ? 1024 : 1;
+    return type == MI355X_TYPE_IQ3_S     ? kIq3sGridSize
+           : type == MI355X_TYPE_IQ3_XXS ? 256
+           : type == MI355X_TYPE_IQ2_S   ? 1024
+                                         : 1;
 }
 template <int TYPE>
 __device__ __forceinline__ void stage_table(const GemmArgs &a, uint2 *tab) {
@@ -574,7 +538,7 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     using Regs = typename RegsOf<TYPE>::T;
     __shared__ uint4 xh0[BM * kGmHalfBytes / 16], xh1[BM * kGmHalfBytes / 16];
     __shared__ uint4 ssum[2][BM * 2];
-    __shared__ float sunit[2][BM];
+    __shared__ float sscale[CONV ? BM : 1], sunit[CONV ? BM : 1];
     __shared__ uint2 tab[gm_table_entries(TYPE)];
 
     const int lane = threadIdx.x & 63;
@@ -614,188 +578,267 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
             }
         }
     }
-    // raw weights of slices (or blocks) 4 half + 2q + h, q = 0, 1
-    auto load_raw = [&](Regs (&r)[NT][2], int b, int half) {
+    // raw weights of slice (or blocks) 4 half + 2q + h of superblock b
+    auto load_raw = [&](Regs (&r)[NT], int b, int half, int q) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
+            if constexpr (Q40) {
+                // rows have an even number of blocks, so a pair exists or not;
+                // past the row (a partial last superblock) the scales are 0
+                // and the codes whatever follows in the buffer
+                const int b0 = 8 * b + 4 * half + 2 * q;
+                const bool in = b0 < a.blocks;
+                const int bc = in ? b0 : 0;
+                r[t].q = ld128(lr[t], static_cast<uint32_t>(128 * b + 16 * h) + 16u * static_cast<uint32_t>(4 * half + 2 * q));
+                const uint32_t F = static_cast<uint32_t>(a.blocks) >> 6;
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                if constexpr (Q40) {
-                    // rows have an even number of blocks: a pair exists or
-                    // not; past the row the scales are 0
-                    const int b0 = 8 * b + 4 * half + 2 * q;
-                    const bool in = b0 < a.blocks;
-                    const int bc = in ? b0 : 0;
-                    r[t][q].q = ld128(lr[t], 16u * static_cast<uint32_t>(bc + h));
-                    const uint32_t F = static_cast<uint32_t>(a.blocks) >> 6;
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const uint32_t be = static_cast<uint32_t>(bc + e);
-                        const uint32_t slot = be < 64 * F ? (be & 63) * F + (be >> 6) : be;  // q4_0_d_slot
-                        r[t][q].d[e] = ld16(lr[t], 16u * static_cast<uint32_t>(a.blocks) + 2 * slot) & (in ? 0xFFFFu : 0u);
-                    }
-                } else {
-                    r[t][q] = Gw<TYPE>::load(lr[t], static_cast<uint32_t>(b), 4 * half + 2 * q + h);
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t be = static_cast<uint32_t>(bc + e);
+                    const uint32_t slot = be < 64 * F ? (be & 63) * F + (be >> 6) : be;  // q4_0_d_slot
+                    r[t].d[e] = ld16(lr[t], 16u * static_cast<uint32_t>(a.blocks) + 2 * slot) & (in ? 0xFFFFu : 0u);
                 }
+            } else {
+                r[t] = Gw<TYPE>::load(lr[t], static_cast<uint32_t>(b), 4 * half + 2 * q + h);
             }
         }
     };
 
-    f32x16 acc[NT][MT], tsum[NT][MT];
+    f32x16 acc[NT][MT];
+    auto clear = [&] {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[t][i] = f32x16{};
+    };
     const int mx = col & 15;  // the rows' slot swizzle (m0 is a multiple of 32)
-
     auto operand = [&](const uint4 *xb, int plane, int run, int tile) {
         const uint4 v = xb[(32 * tile + col) * 32 + 16 * plane + (run ^ mx)];
         return __builtin_bit_cast(f16x8, v);
     };
+    // acc += d * v, in place: sunk to its next use, every block's v would be
+    // live at once
+    auto add_block = [&](f32x16 &c, const f32x16 &v, float d) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) c[k] = fmaf(d, v[k], c[k]);
+        asm volatile("" : "+v"(c));
+    };
 
-    // tsum (+)= this half superblock
-    auto compute = [&](const Regs (&r)[NT][2], const uint4 *xb, int half) {
+    // Operands ahead of their products, of even / odd steps (Q4_0: blocks)
+    u32x4 fw[Q40 ? 1 : NT][2], fl[Q40 ? 1 : NT][2];  // K types: operand and remainder
+    uint2 fe[NT][2][2];                              // codebook entries
+    u32x4 bw[Q40 ? NT : 1][2][2];                    // Q4_0: the block's two operands
+    float bd[NT][2];
+    f32x16 tsum[Q40 ? 1 : NT][Q40 ? 1 : MT];
+    f32x16 vlast;
+    float dlast = 0.f;
+    auto op = [](const u32x4 &v) { return __builtin_bit_cast(f16x8, v); };
+
+    // K types: table entry k, and dword j, of operand step n (q = n / 4, p = n % 4)
+    auto look = [&](const Regs (&r)[2][NT], int n, int t, int k) {
+        if constexpr (!Q40) {
+            if constexpr (Gw<TYPE>::kLooks > 0) fe[t][n & 1][k] = Gw<TYPE>::look(r[n >> 2][t], n & 3, k, tab);
+        }
+    };
+    auto decode = [&](const Regs (&r)[2][NT], int half, int n, int t, int j) {
+        if constexpr (!Q40) {
+            uint32_t hi, lo = 0;
+            Gw<TYPE>::dword(r[n >> 2][t], half, n >> 2, n & 3, j, fe[t][n & 1], hi, lo);
+            fw[t][n & 1][j] = hi;
+            if constexpr (Gw<TYPE>::kWide) fl[t][n & 1][j] = lo;
+        }
+    };
+    // Q4_0: dword j (0..7) of block n
+    auto decode_block = [&](const Regs (&r)[2][NT], int n, int t, int j) {
         if constexpr (Q40) {
+            bw[t][n & 1][j >> 2][j & 3] = q40_dword(r[n >> 1][t], n & 1, j >> 2, j & 3);
+            if (j == 0) bd[t][n & 1] = half_f(r[n >> 1][t].d[n & 1]);
+        }
+    };
+    // first operands of a superblock from its raw weights
+    auto decode_first = [&](const Regs (&r)[2][NT]) {
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                f16x8 w[NT][2][2];
+        for (int t = 0; t < NT; ++t) {
 #pragma unroll
-                for (int t = 0; t < NT; ++t) q40_decode(r[t][q], w[t]);
+            for (int j = 0; j < 8; ++j) decode_block(r, 0, t, j);
+            if constexpr (!Q40) {
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
+                for (int n = 0; n < 2; ++n)
 #pragma unroll
-                    for (int i = 0; i < MT; ++i) {
-                        const int run = 4 * (2 * q + e);
-                        const f16x8 h0 = operand(xb, 0, run + h, i), l0 = operand(xb, 1, run + h, i);
-                        const f16x8 h1 = operand(xb, 0, run + 2 + h, i), l1 = operand(xb, 1, run + 2 + h, i);
+                    for (int k = 0; k < Gw<TYPE>::kLooks; ++k) look(r, n, t, k);
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) {
-                            f32x16 v = {};
-                            v = mfma(h0, w[t][e][0], v);
-                            v = mfma(l0, w[t][e][0], v);
-                            v = mfma(h1, w[t][e][1], v);
-                            v = mfma(l1, w[t][e][1], v);
-                            const float d = half_f(r[t][q].d[e]);
+                for (int j = 0; j < 4; ++j) decode(r, 0, 0, t, j);
+            }
+        }
+    };
+
+    // One half superblock from its raw weights r, its first operands already
+    // decoded; `refill` loads r[0] of the next half once this one's are
+    // decoded, and the last step decodes that half's first operands.
+    auto half_step = [&](Regs (&r)[2][NT], const uint4 *xb, auto HALF, auto refill) {
+        constexpr int half = decltype(HALF)::value;
+        if constexpr (Q40) {
+            f16x8 x[2][4];  // the operands of one (block, row tile), and the next
+            auto read = [&](int u, int k) {
+                const int e = u / MT, i = u % MT;
+                return operand(xb, k & 1, 4 * e + 2 * (k >> 1) + h, i);
+            };
 #pragma unroll
-                            for (int k = 0; k < 16; ++k)
-                                tsum[t][i][k] = half == 0 && q == 0 && e == 0 ? d * v[k] : fmaf(d, v[k], tsum[t][i][k]);
-                            // stays here: sunk to its next use, every block's
-                            // v would be live at once
-                            asm volatile("" : "+v"(tsum[t][i]));
-                        }
+            for (int k = 0; k < 4; ++k) x[0][k] = read(0, k);
+#pragma unroll
+            for (int u = 0; u < 4 * MT; ++u) {
+                const int e = u / MT, i = u % MT;
+                if (u == 2 * MT) refill();  // r[0] is decoded; after the wait for r[1]'s loads at block 1
+                f32x16 v;
+#pragma unroll
+                for (int m = 0; m < 4 * NT; ++m) {
+                    const int t = m >> 2, k = m & 3;
+                    v = mfma(x[u & 1][k], op(bw[t][e & 1][k >> 1]), k == 0 ? f32x16{} : v);
+                    if (u + 1 < 4 * MT && m < 4) x[(u + 1) & 1][m] = read(u + 1, m);
+                    // a quarter of the block sum before this one
+                    f32x16 &c = t ? acc[t - 1][i] : acc[NT - 1][(i + MT - 1) % MT];
+#pragma unroll
+                    for (int z = 4 * k; z < 4 * k + 4; ++z) c[z] = fmaf(dlast, vlast[z], c[z]);
+                    // the next block's operands, 8 NT dwords over its 4 NT MT products
+#pragma unroll
+                    for (int z = 0; z < 8 * NT; ++z)
+                        if (z * MT / 2 == i * 4 * NT + m) decode_block(r, (e + 1) & 3, z >> 3, z & 7);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (k == 3) {
+                        vlast = v;
+                        dlast = bd[t][e & 1];
                     }
                 }
             }
         } else {
-            constexpr int SH = slice_shape(TYPE);
+            constexpr int SH = slice_shape(TYPE), TM = NT * MT, NM = TM * (Gw<TYPE>::kWide ? 3 : 2);
+            constexpr int LOOKS = Gw<TYPE>::kLooks;
+            f16x8 x[2][2 * MT];
+            auto read = [&](int s, int k) { return operand(xb, k & 1, run_of<SH>(2 * (s >> 2) + h, s & 3), k >> 1); };
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                f16x8 wh[NT][4], wl[NT][4];
+            for (int k = 0; k < 2 * MT; ++k) x[0][k] = read(0, k);
 #pragma unroll
-                for (int t = 0; t < NT; ++t) Gw<TYPE>::decode(r[t][q], half, q, tab, wh[t], wl[t]);
+            for (int s = 0; s < 8; ++s) {
+                if (s == 4) refill();  // r[0] is decoded; after the wait for r[1]'s loads in step 3
+                const int n = (s + 1) & 7, nh = s < 7 ? half : 1 - half;
 #pragma unroll
-                for (int p = 0; p < 4; ++p) {
-                    const int run = run_of<SH>(2 * q + h, p);
+                for (int m = 0; m < NM; ++m) {
+                    const int plane = m / TM, i = m / NT % MT, t = m % NT;
+                    const bool first = half == 0 && s == 0 && plane == 0;
+                    tsum[t][i] = mfma(x[s & 1][2 * i + (plane == 1)], op(plane == 2 ? fl[t][s & 1] : fw[t][s & 1]),
+                                      first ? f32x16{} : tsum[t][i]);
+                    if (s < 7 && m < 2 * MT) x[(s + 1) & 1][m] = read(s + 1, m);
+                    // the next step's operands, 4 NT dwords over NM products,
+                    // and the table entries of the one after
 #pragma unroll
-                    for (int i = 0; i < MT; ++i) {
-                        const f16x8 xh = operand(xb, 0, run, i), xl = operand(xb, 1, run, i);
+                    for (int z = 0; z < 4 * NT; ++z)
+                        if (z * NM / (4 * NT) == m) decode(r, nh, n, z >> 2, z & 3);
 #pragma unroll
-                        for (int t = 0; t < NT; ++t) {
-                            f32x16 v = half == 0 && q == 0 && p == 0 ? f32x16{} : tsum[t][i];
-                            v = mfma(xh, wh[t][p], v);
-                            v = mfma(xl, wh[t][p], v);
-                            if constexpr (Gw<TYPE>::kWide) v = mfma(xh, wl[t][p], v);
-                            tsum[t][i] = v;
-                        }
-                    }
+                    for (int z = 0; z < LOOKS * NT; ++z)
+                        if (NM - LOOKS * NT + z == m || (NM < LOOKS * NT && m == NM - 1)) look(r, (s + 2) & 7, z % NT, z / NT);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
         }
     };
-    // acc += unit_m * (d * tsum - dmin * mins . sums)
-    auto finish = [&](const Regs (&r)[NT][2], int par) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            float un[16];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const float4 u = *reinterpret_cast<const float4 *>(&sunit[par][32 * i + 8 * g + 4 * h]);
-                un[4 * g] = u.x;
-                un[4 * g + 1] = u.y;
-                un[4 * g + 2] = u.z;
-                un[4 * g + 3] = u.w;
-            }
+    // K types, end of a superblock: acc += d * tsum - dmin * mins . sums
+    auto finish = [&](const Regs (&r)[NT], int par) {
+        if constexpr (!Q40) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                if constexpr (Q40) {
+                const float d = Gw<TYPE>::d(r[t]);
+                if constexpr (Gw<TYPE>::kMins) {
+                    const f16x8 mins = k4_mins(r[t].hd);
+                    const float dm = -32.0f * half_f(r[t].hd[0] >> 16);
 #pragma unroll
-                    for (int k = 0; k < 16; ++k) acc[t][i][k] = fmaf(un[k], tsum[t][i][k], acc[t][i][k]);
-                } else {
-                    const float d = Gw<TYPE>::d(r[t][0]);
-                    if constexpr (Gw<TYPE>::kMins) {
+                    for (int i = 0; i < MT; ++i) {
                         // operand halves h = 0, 1: the sums' hi and lo planes
                         const f16x8 s = __builtin_bit_cast(f16x8, ssum[par][(32 * i + col) * 2 + h]);
-                        const f32x16 mm = mfma(s, k4_mins(r[t][0].hd), f32x16{});
-                        const float dm = -32.0f * half_f(r[t][0].hd[0] >> 16);
+                        const f32x16 mm = mfma(s, mins, f32x16{});
 #pragma unroll
-                        for (int k = 0; k < 16; ++k)
-                            acc[t][i][k] = fmaf(un[k], fmaf(dm, mm[k], d * tsum[t][i][k]), acc[t][i][k]);
+                        for (int k = 0; k < 16; ++k) acc[t][i][k] += fmaf(dm, mm[k], d * tsum[t][i][k]);
                         __builtin_amdgcn_sched_barrier(0);
-                    } else {
-#pragma unroll
-                        for (int k = 0; k < 16; ++k) acc[t][i][k] = fmaf(un[k], d * tsum[t][i][k], acc[t][i][k]);
                     }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) add_block(acc[t][i], tsum[t][i], d);
                 }
             }
+        }
+    };
+    // Q4_0: the last block sum
+    auto flush = [&] {
+        if constexpr (Q40) {
+            add_block(acc[NT - 1][MT - 1], vlast, dlast);
+            vlast = f32x16{};
+            dlast = 0.f;
         }
     };
     // segment `seg` to out (CONV: added to the segments before it)
-    auto store = [&](int seg) {
+    auto store = [&](int seg, auto unit) {
         float *out = a.out + (CONV ? 0 : seg * a.seg_stride);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int64_t n = n0 + 32 * t + col;
-            if (n >= a.N) continue;
+        for (int i = 0; i < MT; ++i) {
 #pragma unroll
-            for (int i = 0; i < MT; ++i) {
+            for (int k = 0; k < 16; ++k) {
+                const int m = m0 + 32 * i + 8 * (k >> 2) + 4 * h + (k & 3);
+                if (m >= a.M) continue;
+                const float u = unit(m);
 #pragma unroll
-                for (int k = 0; k < 16; ++k) {
-                    const int m = m0 + 32 * i + 8 * (k >> 2) + 4 * h + (k & 3);
-                    if (m < a.M) {
-                        float *p = out + m * a.out_stride + n;
-                        if constexpr (CONV) *p = seg == 0 ? acc[t][i][k] : *p + acc[t][i][k];
-                        else *p = acc[t][i][k];
-                    }
+                for (int t = 0; t < NT; ++t) {
+                    const int64_t n = n0 + 32 * t + col;
+                    if (n >= a.N) continue;
+                    float *p = out + m * a.out_stride + n;
+                    const float v = u * acc[t][i][k];
+                    if constexpr (CONV) *p = seg == 0 ? v : *p + v;
+                    else *p = v;
                 }
             }
         }
     };
 
+    using H0 = std::integral_constant<int, 0>;
+    using H1 = std::integral_constant<int, 1>;
     stage_table<TYPE>(a, tab);
+    vlast = f32x16{};
 
     if constexpr (CONV) {
+        const bool al16 = a.x_al16 != 0;
+        auto load = [&](int r, int b) {
+            const int64_t left = a.K - 256 * static_cast<int64_t>(b);
+            return load_x4(a.x + (m0 + r) * a.x_stride + 256 * static_cast<int64_t>(b), 4 * lane,
+                           static_cast<int>(left < 256 ? left : 256), al16);
+        };
+        for (int r = wave; r < BM && m0 + r < a.M; r += kGmWaves) {
+            float m = 0.f, u;
+            for (int b = 0; b < a.B; ++b) m = fmaxf(m, abs_max4(load(r, b)));
+            const float s = row_scale(wave_max(m), u);
+            if (lane == 0) {
+                sscale[r] = s;
+                sunit[r] = u;
+            }
+        }
         for (int seg = 0; seg < a.nseg; ++seg) {
             const int b0 = seg * a.per_seg, b1 = min(b0 + a.per_seg, a.B);
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int i = 0; i < MT; ++i) acc[t][i] = f32x16{};
+            clear();
+            Regs r[2][NT];
             for (int b = b0; b < b1; ++b) {
-                Regs r0[NT][2], r1[NT][2];
-                load_raw(r0, b, 0);
-                load_raw(r1, b, 1);
-                __syncthreads();  // the previous superblock's operands are read
-                const int64_t left = a.K - 256 * static_cast<int64_t>(b);
-                for (int r = wave; r < BM && m0 + r < a.M; r += kGmWaves) {
-                    const XPlanes c = convert_superblock(a.x + (m0 + r) * a.x_stride + 256 * static_cast<int64_t>(b),
-                                                         static_cast<int>(left < 256 ? left : 256), a.x_al16 != 0, lane);
-                    store_superblock(c, r, lane, reinterpret_cast<uint8_t *>(xh0) + kGmHalfBytes * r,
-                                     reinterpret_cast<uint8_t *>(xh1) + kGmHalfBytes * r,
-                                     reinterpret_cast<_Float16 *>(ssum[0]) + 16 * r);
-                    if (lane == 0) sunit[0][r] = c.unit;
-                }
+                load_raw(r[0], b, 0, 0);
+                load_raw(r[1], b, 0, 1);
+                __syncthreads();  // scales written; the previous superblock's operands are read
+                for (int row = wave; row < BM && m0 + row < a.M; row += kGmWaves)
+                    store_superblock(convert_superblock(load(row, b), sscale[row]), row, lane,
+                                     reinterpret_cast<uint8_t *>(xh0) + kGmHalfBytes * row,
+                                     reinterpret_cast<uint8_t *>(xh1) + kGmHalfBytes * row,
+                                     reinterpret_cast<_Float16 *>(ssum[0]) + 16 * row);
                 __syncthreads();
-                compute(r0, xh0, 0);
-                compute(r1, xh1, 1);
-                finish(r1, 0);
+                decode_first(r);
+                half_step(r, xh0, H0{}, [&] { load_raw(r[0], b, 1, 0); });
+                load_raw(r[1], b, 1, 1);
+                half_step(r, xh1, H1{}, [&] {});
+                finish(r[1], 0);
             }
-            store(seg);
+            flush();
+            store(seg, [&](int m) { return sunit[m - m0]; });
         }
     } else {
         const int seg = blockIdx.y;
@@ -803,47 +846,42 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
         auto half_src = [&](int b, int half) {
             return a.planes + (static_cast<int64_t>(2 * b + half) * a.Mp + m0) * kGmHalfBytes;
         };
-        // sums and units of superblock b: threads 0 .. 2 BM - 1 and 0 .. BM - 1
-        auto load_tail = [&](int b, uint4 &s, float &u) {
-            if (threadIdx.x < 2 * BM)
+        constexpr bool MINS = TYPE == MI355X_TYPE_Q4_K || TYPE == MI355X_TYPE_Q5_K;
+        // sums of superblock b (types with mins): threads 0 .. 2 BM - 1
+        auto load_sums = [&](int b, uint4 &s) {
+            if (MINS && threadIdx.x < 2 * BM)
                 s = reinterpret_cast<const uint4 *>(a.sums)[(static_cast<int64_t>(b) * a.Mp + m0) * 2 + threadIdx.x];
-            if (threadIdx.x < BM) u = a.unit[static_cast<int64_t>(b) * a.Mp + m0 + threadIdx.x];
         };
-        auto put_tail = [&](int par, const uint4 &s, float u) {
-            if (threadIdx.x < 2 * BM) ssum[par][threadIdx.x] = s;
-            if (threadIdx.x < BM) sunit[par][threadIdx.x] = u;
+        auto put_sums = [&](int par, const uint4 &s) {
+            if (MINS && threadIdx.x < 2 * BM) ssum[par][threadIdx.x] = s;
         };
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int i = 0; i < MT; ++i) acc[t][i] = f32x16{};
+        clear();
         uint4 s = make_uint4(0, 0, 0, 0);
-        float u = 0.f;
-        Regs r[NT][2], rn[NT][2];
+        Regs r[2][NT];
         copy_planes<BM>(half_src(b0, 0), xh0, wave, lane);
-        load_tail(b0, s, u);
-        load_raw(r, b0, 0);
-        put_tail(b0 & 1, s, u);
+        load_sums(b0, s);
+        load_raw(r[0], b0, 0, 0);
+        put_sums(b0 & 1, s);
         gm_barrier();
+        decode_first(r);
         for (int b = b0; b < b1; ++b) {
-            const bool more = b + 1 < b1;
+            const int bn = b + 1 < b1 ? b + 1 : b;  // the last superblock's look-ahead reads itself again
             copy_planes<BM>(half_src(b, 1), xh1, wave, lane);
-            load_raw(rn, b, 1);
-            __builtin_amdgcn_sched_barrier(0);  // the next half's loads go out before this half's work
-            compute(r, xh0, 0);
+            load_raw(r[1], b, 0, 1);
+            __builtin_amdgcn_sched_barrier(0);  // the loads go out before this half's work
+            half_step(r, xh0, H0{}, [&] { load_raw(r[0], b, 1, 0); });
             gm_barrier();
-            if (more) {
-                copy_planes<BM>(half_src(b + 1, 0), xh0, wave, lane);
-                load_tail(b + 1, s, u);
-                load_raw(r, b + 1, 0);
-            }
+            copy_planes<BM>(half_src(bn, 0), xh0, wave, lane);
+            load_sums(bn, s);
+            load_raw(r[1], b, 1, 1);
             __builtin_amdgcn_sched_barrier(0);
-            compute(rn, xh1, 1);
-            finish(rn, b & 1);
-            if (more) put_tail((b + 1) & 1, s, u);
+            half_step(r, xh1, H1{}, [&] { load_raw(r[0], bn, 0, 0); });
+            finish(r[1], b & 1);
+            put_sums((b + 1) & 1, s);
             gm_barrier();
         }
-        store(seg);
+        flush();
+        store(seg, [&](int m) { return a.unit[m]; });
     }
 }
 
@@ -960,7 +998,7 @@ int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
         }
         const size_t planes = static_cast<size_t>(g.B) * 2 * g.Mp * kGmHalfBytes;
         const size_t sums = static_cast<size_t>(g.B) * g.Mp * 32;
-        const size_t units = align256(static_cast<size_t>(g.B) * g.Mp * 4);
+        const size_t units = align256(static_cast<size_t>(g.Mp) * 4);
         const size_t part = g.nseg > 1 ? static_cast<size_t>(g.nseg) * M * a.N * 4 : 0;
         const size_t need = planes + align256(sums) + units + part;
         if (ctx->gemm_bytes < need) {
@@ -979,9 +1017,8 @@ int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
         g.out = g.nseg > 1 ? partial : y;
         g.out_stride = g.nseg > 1 ? a.N : y_stride;
         g.seg_stride = static_cast<int64_t>(M) * a.N;
-        const int64_t tasks = static_cast<int64_t>(M) * g.B;
-        hipLaunchKernelGGL(gemm_planes_kernel, dim3(static_cast<unsigned>((tasks + 3) / 4)), dim3(256), 0, ctx->stream,
-                           g.x, x_stride, a.K, g.x_al16, M, g.Mp, g.B, p, const_cast<_Float16 *>(g.sums),
+        hipLaunchKernelGGL(gemm_planes_kernel, dim3(static_cast<unsigned>(M)), dim3(kPlThreads), 0, ctx->stream, g.x,
+                           x_stride, a.K, g.x_al16, g.Mp, g.B, p, const_cast<_Float16 *>(g.sums),
                            const_cast<float *>(g.unit));
         MI355X_HIP(hipGetLastError());
         hipLaunchKernelGGL(k, dim3(grid_x, static_cast<unsigned>(g.nseg)), dim3(kGmThreads), 0, ctx->stream, g);
