@@ -174,7 +174,9 @@ __device__ __forceinline__ void kq_row_group(const KqArgs &a, int64_t g, typenam
 // wavefronts, one workgroup per CU): workgroup b takes a contiguous block of
 // ceil(groups / grid) row groups, its wavefronts interleaved in it, so every
 // SIMD gets the same number of rows within one.
-template <int TYPE, int R, int NIT, bool DG, bool PF, int NT>
+// With ANYX the activations are read as the caller has them (BF16, or f32 off
+// a 16-byte boundary).
+template <int TYPE, int R, int NIT, bool DG, bool PF, int NT, bool ANYX = false>
 __global__ __launch_bounds__(NT) void gemv_kq_kernel(KqArgs a) {
     using K = Kq<TYPE>;
     // the codebook in static LDS (its address is known when the lookups are
@@ -210,15 +212,13 @@ __global__ __launch_bounds__(NT) void gemv_kq_kernel(KqArgs a) {
     // 1. activation loads for staging: runs r = threadIdx.x + NT k of
     // the chunk (8 values each)
     const int nruns = 32 * a.nb;
-    const float *xc = a.x + static_cast<int64_t>(a.b0) * 256;
     float4 xv[kRuns][2];
 #pragma unroll
     for (int k = 0; k < kRuns; ++k) {
         if (k == 0 || NT * k < nruns) {
             const int r = static_cast<int>(threadIdx.x) + NT * k;
-            const float4 *src = reinterpret_cast<const float4 *>(xc + 8 * (r < nruns ? r : nruns - 1));
-            xv[k][0] = src[0];
-            xv[k][1] = src[1];
+            load_x8(a.x, ANYX ? a.x_kind : static_cast<int>(kXF32),
+                    static_cast<int64_t>(a.b0) * 256 + 8 * (r < nruns ? r : nruns - 1), xv[k][0], xv[k][1]);
         }
     }
     GridRegs<TYPE, NT> gr;
@@ -658,22 +658,37 @@ kq_kernel_fn pick_dg(int R, int nit, bool wide) {
     }
 }
 
+template <int TYPE, bool DG>
+kq_kernel_fn pick_any(int nit) {
+    switch (nit) {
+    case 1: return gemv_kq_kernel<TYPE, 1, 1, DG, false, kThreads, true>;
+    case 2: return gemv_kq_kernel<TYPE, 1, 2, DG, false, kThreads, true>;
+    case 3: return gemv_kq_kernel<TYPE, 1, 3, DG, false, kThreads, true>;
+    case 4: return gemv_kq_kernel<TYPE, 1, 4, DG, false, kThreads, true>;
+    case 5: return gemv_kq_kernel<TYPE, 1, 5, DG, false, kThreads, true>;
+    case 6: return gemv_kq_kernel<TYPE, 1, 6, DG, false, kThreads, true>;
+    case 7: return gemv_kq_kernel<TYPE, 1, 7, DG, false, kThreads, true>;
+    default: return gemv_kq_kernel<TYPE, 1, 8, DG, false, kThreads, true>;
+    }
+}
+
 template <int TYPE>
-kq_kernel_fn pick(int R, int nit, bool dg, bool pf, bool wide) {
+kq_kernel_fn pick(int R, int nit, bool dg, bool pf, bool wide, bool any) {
+    if (any) return dg ? pick_any<TYPE, true>(nit) : pick_any<TYPE, false>(nit);
     if (pf) return dg ? pick_dg<TYPE, true, true>(R, nit, wide) : pick_dg<TYPE, false, true>(R, nit, wide);
     return dg ? pick_dg<TYPE, true, false>(R, nit, wide) : pick_dg<TYPE, false, false>(R, nit, wide);
 }
 
-kq_kernel_fn pick_kernel(int type, int R, int nit, bool dg, bool pf, bool wide) {
+kq_kernel_fn pick_kernel(int type, int R, int nit, bool dg, bool pf, bool wide, bool any) {
     switch (type) {
-    case MI355X_TYPE_Q4_K: return pick<MI355X_TYPE_Q4_K>(R, nit, dg, pf, wide);
-    case MI355X_TYPE_Q5_K: return pick<MI355X_TYPE_Q5_K>(R, nit, dg, pf, wide);
-    case MI355X_TYPE_Q3_K: return pick<MI355X_TYPE_Q3_K>(R, nit, dg, pf, wide);
-    case MI355X_TYPE_Q6_K: return pick<MI355X_TYPE_Q6_K>(R, nit, dg, pf, wide);
-    case MI355X_TYPE_IQ4_XS: return pick<MI355X_TYPE_IQ4_XS>(R, nit, dg, pf, wide);
-    case MI355X_TYPE_IQ3_S: return pick<MI355X_TYPE_IQ3_S>(R, nit, dg, pf, wide);
-    case MI355X_TYPE_IQ3_XXS: return pick<MI355X_TYPE_IQ3_XXS>(R, nit, dg, pf, wide);
-    case MI355X_TYPE_IQ2_S: return pick<MI355X_TYPE_IQ2_S>(R, nit, dg, pf, wide);
+    case MI355X_TYPE_Q4_K: return pick<MI355X_TYPE_Q4_K>(R, nit, dg, pf, wide, any);
+    case MI355X_TYPE_Q5_K: return pick<MI355X_TYPE_Q5_K>(R, nit, dg, pf, wide, any);
+    case MI355X_TYPE_Q3_K: return pick<MI355X_TYPE_Q3_K>(R, nit, dg, pf, wide, any);
+    case MI355X_TYPE_Q6_K: return pick<MI355X_TYPE_Q6_K>(R, nit, dg, pf, wide, any);
+    case MI355X_TYPE_IQ4_XS: return pick<MI355X_TYPE_IQ4_XS>(R, nit, dg, pf, wide, any);
+    case MI355X_TYPE_IQ3_S: return pick<MI355X_TYPE_IQ3_S>(R, nit, dg, pf, wide, any);
+    case MI355X_TYPE_IQ3_XXS: return pick<MI355X_TYPE_IQ3_XXS>(R, nit, dg, pf, wide, any);
+    case MI355X_TYPE_IQ2_S: return pick<MI355X_TYPE_IQ2_S>(R, nit, dg, pf, wide, any);
     default: return nullptr;
     }
 }
@@ -1207,12 +1222,23 @@ int launch_gemv_kquant(mi355x_ctx *ctx, const GemvArgs &a) {
     if (grid_words(a.type) > 0 && a.type != MI355X_TYPE_IQ3_S && !grid)
         return set_error(MI355X_EUNSUPPORTED, "grid table not installed for this IQ type");
 
-    // activations as 16-byte aligned f32 (bf16 and unaligned inputs go
-    // through the context's activation buffer; the context lock keeps the
-    // buffer in place from the conversion to the last launch that reads it)
+    // The one-row row kernels read x as the caller has it, BF16 or unaligned
+    // (Q3_K 3001x2816 with BF16 activations 4.2 us, with a widening launch
+    // before the GEMV 7.6; a kernel of its own, as the choice of load costs
+    // aligned f32 0.5 us at Q4_K 14336x4096).  The others take 16-byte aligned
+    // f32, so such inputs go through the context's activation buffer (the
+    // context lock keeps the buffer in place from the conversion to the last
+    // launch that reads it).
+    const bool x_al16 = (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
+    const bool plain_f32 = !a.x_bf16 && x_al16;
+    const bool any_x = !plain_f32 && ctx->kernel_variant != MI355X_VARIANT_GGML_Q8 &&
+                       (ctx->kernel_variant == MI355X_VARIANT_EXACT_F32 ||
+                        (ctx->form_override != MI355X_FORM_PIPE && ctx->form_override != MI355X_FORM_KSPLIT)) &&
+                       ctx->rows_override != 2 && ctx->prefetch_override != 1;
+    const int x_kind = a.x_bf16 ? (x_al16 ? kXBf16 : kXBf16Any) : (x_al16 ? kXF32 : kXF32Any);
     const float *x = static_cast<const float *>(a.x);
     std::unique_lock<std::mutex> lk(ctx->mu, std::defer_lock);
-    if (a.x_bf16 || (reinterpret_cast<uintptr_t>(a.x) & 15) != 0) {
+    if (!plain_f32 && !any_x) {
         lk.lock();
         const size_t need = static_cast<size_t>(a.K) * sizeof(float);
         if (ctx->xconv_bytes < need) {
@@ -1349,11 +1375,11 @@ int launch_gemv_kquant(mi355x_ctx *ctx, const GemvArgs &a) {
         int R = 1;
         if (ctx->rows_override == 1 || (ctx->rows_override == 2 && nit <= max_nit_r2(a.type))) R = ctx->rows_override;
         const bool pf = R == 1 && ctx->prefetch_override == 1;
-        const bool wide = (a.type == MI355X_TYPE_IQ3_S || a.type == MI355X_TYPE_IQ2_S) && dg && !pf && R == 1 &&
+        const bool wide = (a.type == MI355X_TYPE_IQ3_S || a.type == MI355X_TYPE_IQ2_S) && dg && !pf && R == 1 && !any_x &&
                           nit <= kWideMaxNit && nb >= 32 &&
                           !ctx->ov_open;
         const int nt = wide ? kWideThreads : kThreads;
-        const kq_kernel_fn k = pick_kernel(a.type, R, nit, dg, pf, wide);
+        const kq_kernel_fn k = pick_kernel(a.type, R, nit, dg, pf, wide, any_x);
         const int64_t n_groups = (a.N + R - 1) / R;
         // dynamic LDS: the records (the codebook is the kernel's static LDS)
         const size_t lds = dg ? dg_lds_bytes(nb) : x_lds_bytes(nb);
@@ -1372,7 +1398,7 @@ int launch_gemv_kquant(mi355x_ctx *ctx, const GemvArgs &a) {
         int64_t wgs = std::min<int64_t>((n_groups + nw - 1) / nw, static_cast<int64_t>(ctx->num_cus) * per_cu);
         if (ctx->grid_override > 0) wgs = std::min<int64_t>(wgs, ctx->grid_override);
         KqArgs args{a.W, a.N, row_bytes, static_cast<int>(B), static_cast<int>(b0), nb, x, a.y, b0 > 0 ? 1 : 0,
-                    grid};
+                    grid, any_x ? x_kind : static_cast<int>(kXF32)};
         hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(std::max<int64_t>(wgs, 1))), dim3(nt), lds,
                            ctx->stream, args);
         MI355X_HIP(hipGetLastError());

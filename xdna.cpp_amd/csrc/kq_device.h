@@ -34,7 +34,37 @@ struct KqArgs {
     float *y;
     int accumulate;
     const uint32_t *grid;  // device codebook (IQ3_XXS, IQ2_S), else null
+    int x_kind;            // row kernels: how x is read (XKind); 0 elsewhere
 };
+// Activations as the caller has them: f32 or BF16 (widened exactly), on a
+// 16-byte boundary or not.
+enum XKind { kXF32 = 0, kXF32Any = 1, kXBf16 = 2, kXBf16Any = 3 };
+
+__device__ __forceinline__ float4 bf16x4_to_float4(uint32_t a, uint32_t b) {
+    return make_float4(__builtin_bit_cast(float, a << 16), __builtin_bit_cast(float, a & 0xFFFF0000u),
+                       __builtin_bit_cast(float, b << 16), __builtin_bit_cast(float, b & 0xFFFF0000u));
+}
+// the 8 values from value i of x (i a multiple of 8)
+__device__ __forceinline__ void load_x8(const void *x, int kind, int64_t i, float4 &lo, float4 &hi) {
+    if (kind == kXF32) {
+        const float4 *p = reinterpret_cast<const float4 *>(static_cast<const float *>(x) + i);
+        lo = p[0];
+        hi = p[1];
+    } else if (kind == kXF32Any) {
+        const float *p = static_cast<const float *>(x) + i;
+        lo = make_float4(p[0], p[1], p[2], p[3]);
+        hi = make_float4(p[4], p[5], p[6], p[7]);
+    } else {
+        const uint16_t *p = static_cast<const uint16_t *>(x) + i;
+        uint4 v;
+        if (kind == kXBf16) v = *reinterpret_cast<const uint4 *>(p);
+        else
+            v = make_uint4(p[0] | static_cast<uint32_t>(p[1]) << 16, p[2] | static_cast<uint32_t>(p[3]) << 16,
+                           p[4] | static_cast<uint32_t>(p[5]) << 16, p[6] | static_cast<uint32_t>(p[7]) << 16);
+        lo = bf16x4_to_float4(v.x, v.y);
+        hi = bf16x4_to_float4(v.z, v.w);
+    }
+}
 
 __device__ __forceinline__ float byte_f(uint32_t w, int t) { return static_cast<float>((w >> (8 * t)) & 0xFFu); }
 
