@@ -290,7 +290,10 @@ MI355X_API int mi355x_gemv_bf16(mi355x_ctx *ctx, int type, const void *W, int64_
  * weights: activations as two f16 planes (22 bits), products exact, f32 sums
  * (one launch that splits the activations into a context buffer, one product
  * launch, and one that adds the partial sums where K is split; IQ3_XXS and
- * IQ2_S with grids of magnitudes up to 66).  Fewer Q4_0 activations with the
+ * IQ2_S with grids of magnitudes up to 66).  A few activations (2 to 8, as
+ * many as fit the LDS) of the other types run in one launch with the one-row
+ * kernels' digit arithmetic on the integer matrix cores, where those kernels
+ * use it and K <= 16384.  Fewer Q4_0 activations with the
  * digit-plane arithmetic, rows a multiple of 256 values and 16-byte aligned
  * weights: up to 8 per pass (one staging launch into a context buffer, one
  * batched launch).  Other cases:

@@ -1205,7 +1205,52 @@ kq_q8k_fn pick_q8k_kernel(int type, int nit) {
     }
 }
 
+// equal chunks of at most kChunkBlocks superblocks
+int64_t chunk_blocks(int64_t B) {
+    const int64_t n = (B + kChunkBlocks - 1) / kChunkBlocks;
+    return (B + n - 1) / n;
+}
+
+// Default forms (variant and form AUTO), from sweeps of the headline
+// shapes on MI355X (us, 14336x4096 / 4096x14336; 8192x8192 for IQ;
+// boxes differ by up to ~0.4 us):
+//  * every type: digit rows, one row per wavefront step, each step's
+//    registers refilled with the next row group's step right after its
+//    decode (Q3_K 9.1 / 10.9, Q4_K 7.9 / 9.3, Q5_K 9.8 / 11.1, Q6_K
+//    11.1 / 13.2, IQ4_XS 10.7, IQ3_S 11.4, IQ2_S 10.6, IQ3_XXS 9.8; the
+//    next group loaded after the whole decode: 10.2 / 11.5, 8.3 / 9.9,
+//    9.8 / 11.4, 11.2 / 13.3, 11.0, 11.6 (two rows per step), 10.8 (two
+//    rows), 10.0);
+//  * IQ4_XS only up to four steps and the codebook types only up to
+//    four steps and N >= 4096 (f32 rows otherwise): table-driven sign
+//    application and dot4 products cost fewer VALU instructions than the
+//    f32 decode (f32 14.0 / 12.2 / 12.7 for IQ3_S / IQ3_XXS / IQ2_S).
+// Prefetch (a second register set for the next row group, requested
+// before the current one's decode) is off by default: the refill gives
+// the loads the same head start without the second set (Q3_K 9.2 / 10.9
+// with prefetch).
+bool dg_rows_auto(int type, int64_t N, int nit) {
+    switch (type) {
+    case MI355X_TYPE_Q3_K:
+    case MI355X_TYPE_Q4_K:
+    case MI355X_TYPE_Q5_K:
+    case MI355X_TYPE_Q6_K: return true;
+    case MI355X_TYPE_IQ4_XS: return nit <= 4;
+    case MI355X_TYPE_IQ3_S:
+    case MI355X_TYPE_IQ3_XXS:
+    case MI355X_TYPE_IQ2_S: return nit <= max_nit_r2(type) && N >= 4096;
+    default: return false;
+    }
+}
+
 }  // namespace
+
+bool kq_digit_rows(const mi355x_ctx *ctx, int type, int64_t N, int64_t K) {
+    if (ctx->kernel_variant == MI355X_VARIANT_DIGITS) return true;
+    if (ctx->kernel_variant != MI355X_VARIANT_AUTO) return false;
+    const int64_t nb = chunk_blocks(K / 256);
+    return dg_rows_auto(type, N, static_cast<int>((nb + kBlocksPerStep - 1) / kBlocksPerStep));
+}
 
 int launch_gemv_kquant(mi355x_ctx *ctx, const GemvArgs &a) {
     const KqLayout L = kq_layout(a.type);
@@ -1287,40 +1332,9 @@ int launch_gemv_kquant(mi355x_ctx *ctx, const GemvArgs &a) {
         return MI355X_OK;
     }
 
-    const bool grid_type = a.type == MI355X_TYPE_IQ3_S || a.type == MI355X_TYPE_IQ3_XXS || a.type == MI355X_TYPE_IQ2_S;
     const bool dg_forced = ctx->kernel_variant == MI355X_VARIANT_DIGITS;
 
-    // equal chunks of at most kChunkBlocks superblocks
-    const int64_t n_chunks = (B + kChunkBlocks - 1) / kChunkBlocks;
-    const int64_t per_chunk = (B + n_chunks - 1) / n_chunks;
-    // Default forms (variant and form AUTO), from sweeps of the BASELINE
-    // shapes on MI355X (us, 14336x4096 / 4096x14336; 8192x8192 for IQ;
-    // boxes differ by up to ~0.4 us):
-    //  * every type: digit rows, one row per wavefront step, each step's
-    //    registers refilled with the next row group's step right after its
-    //    decode (Q3_K 9.1 / 10.9, Q4_K 7.9 / 9.3, Q5_K 9.8 / 11.1, Q6_K
-    //    11.1 / 13.2, IQ4_XS 10.7, IQ3_S 11.4, IQ2_S 10.6, IQ3_XXS 9.8; the
-    //    next group loaded after the whole decode: 10.2 / 11.5, 8.3 / 9.9,
-    //    9.8 / 11.4, 11.2 / 13.3, 11.0, 11.6 (two rows per step), 10.8 (two
-    //    rows), 10.0);
-    //  * IQ4_XS only up to four steps and the codebook types only up to
-    //    four steps and N >= 4096 (f32 rows otherwise): table-driven sign
-    //    application and dot4 products cost fewer VALU instructions than the
-    //    f32 decode (f32 14.0 / 12.2 / 12.7 for IQ3_S / IQ3_XXS / IQ2_S).
-    // Prefetch (a second register set for the next row group, requested
-    // before the current one's decode) is off by default: the refill gives
-    // the loads the same head start without the second set (Q3_K 9.2 / 10.9
-    // with prefetch).
-    auto dg_rows_auto = [&](int nit) {
-        switch (a.type) {
-        case MI355X_TYPE_Q3_K:
-        case MI355X_TYPE_Q4_K:
-        case MI355X_TYPE_Q5_K:
-        case MI355X_TYPE_Q6_K: return true;
-        case MI355X_TYPE_IQ4_XS: return nit <= 4;
-        default: return grid_type && nit <= max_nit_r2(a.type) && a.N >= 4096;
-        }
-    };
+    const int64_t per_chunk = chunk_blocks(B);
     for (int64_t b0 = 0; b0 < B; b0 += per_chunk) {
         const int nb = static_cast<int>(std::min<int64_t>(per_chunk, B - b0));
         const int nit = (nb + kBlocksPerStep - 1) / kBlocksPerStep;
@@ -1370,7 +1384,7 @@ int launch_gemv_kquant(mi355x_ctx *ctx, const GemvArgs &a) {
             MI355X_HIP(hipGetLastError());
             continue;
         }
-        const bool dg_auto = ctx->kernel_variant == MI355X_VARIANT_AUTO && dg_rows_auto(nit);
+        const bool dg_auto = ctx->kernel_variant == MI355X_VARIANT_AUTO && dg_rows_auto(a.type, a.N, nit);
         const bool dg = dg_forced || dg_auto;
         int R = 1;
         if (ctx->rows_override == 1 || (ctx->rows_override == 2 && nit <= max_nit_r2(a.type))) R = ctx->rows_override;

@@ -144,6 +144,13 @@ bool q4_0_q8_supports(const mi355x_ctx *ctx, const GemvArgs &a);
 int launch_gemv_q4_0_q8(mi355x_ctx *ctx, const GemvArgs &a);
 int launch_gemv_q4_0_st(mi355x_ctx *ctx, const GemvArgs &a);
 int launch_gemv_kquant(mi355x_ctx *ctx, const GemvArgs &a);
+// Whether a GEMV of this type and size runs in digit arithmetic (16-bit
+// activations) in the context's variant.
+bool kq_digit_rows(const mi355x_ctx *ctx, int type, int64_t N, int64_t K);
+// A few activations of a K/IQ matrix in one launch (digit arithmetic), where
+// that is the fastest form for these sizes.
+bool kq_mx_takes(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M);
+int launch_gemv_kq_mx(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int M);
 
 // Prepack kernels: byte-range scatter/gather between ggml and resident order.
 int launch_prepack_scatter(mi355x_ctx *ctx, int type, int64_t N, int64_t K, uint8_t *packed,

@@ -925,7 +925,7 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
                                                       ": the grid is not on this context yet (one mi355x_gemv of "
                                                       "this type on the context first)");
     }
-    // many activations: the matrix cores (every type)
+    // the matrix cores: a few activations of a K/IQ type, many of any type
     if (ctx && M >= 2 && N > 0 && K > 0 && W && x && y && (reinterpret_cast<uintptr_t>(W) & 1) == 0 &&
         mi355x_type_ready(type)) {
         uint64_t total = 0;
@@ -937,6 +937,7 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
             if (rc) return rc;
         }
         GemvArgs a{type, static_cast<const uint8_t *>(W), N, K, x, false, y};
+        if (kq_mx_takes(ctx, a, M)) return launch_gemv_kq_mx(ctx, a, x_stride, y_stride, static_cast<int>(M));
         if (gemm_batched_supports(ctx, a, M)) return launch_gemm_batched(ctx, a, x_stride, y_stride, M, noalloc);
     }
     // Q4_0 digit-plane arithmetic: up to q4_0_mb_capacity() activations per
