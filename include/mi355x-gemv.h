@@ -285,10 +285,12 @@ MI355X_API int mi355x_gemv_bf16(mi355x_ctx *ctx, int type, const void *W, int64_
  * y + m*y_stride floats); the M-row case the reference admits for weights in
  * its own buffer type and computes as M sequential GEMVs
  * (src/ggml-xdna.cpp:110-112, 287-296).  In the variants AUTO and DIGITS many
- * activations (M >= 16 for Q4_0 with an even number of blocks per row, M >= 4
- * for the other types) run on the matrix cores, up to 512 per pass over the
- * weights: activations as two f16 planes (22 bits), products exact, f32 sums
- * (one launch that splits the activations into a context buffer, one product
+ * activations (for Q4_0 with an even number of blocks per row M >= 17, from 2^25
+ * weights M >= 12; for the other types M >= 4, or 5 where the one-row kernels
+ * sum a codebook type in f32) run on the matrix cores, up to 512 per pass over
+ * the weights: activations as two f16 planes (22 bits), products exact, f32
+ * sums (one launch that splits the activations into the context's 64 MiB
+ * workspace, allocated with the context and freed with it, one product
  * launch, and one that adds the partial sums where K is split; IQ3_XXS and
  * IQ2_S with grids of magnitudes up to 66).  A few activations (2 to 8, as
  * many as fit the LDS) of the other types run in one launch with the one-row
@@ -306,10 +308,9 @@ MI355X_API int mi355x_gemv_batched(mi355x_ctx *ctx, int type, const void *W, int
 /* Allocation-free form of mi355x_gemv_batched, for callers that cannot call
  * hipMalloc (code under HIP graph capture, tight serving loops, harnesses
  * that forbid it).  No counterpart in the reference.  Same arguments and the
- * same outputs, bit for bit; the matrix-core form converts activations in
- * each workgroup and takes the segments of K one after another; the K-split
- * batched form keeps its activation tiles in the library's static device
- * scratch of
+ * same outputs, bit for bit; the matrix-core forms are the same launches (the
+ * workspace is the context's from its creation); the K-split batched form
+ * keeps its activation tiles in the library's static device scratch of
  * MI355X_NOALLOC_SCRATCH_BYTES (336 KiB per device, held until the process
  * ends; enough for 8 activations of K = 16384 per pass, the most the form
  * stages) instead of a context buffer grown with hipMalloc.  Every call on

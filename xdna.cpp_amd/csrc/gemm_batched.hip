@@ -74,10 +74,6 @@ struct GemmArgs {
     const uint8_t *planes;  // [superblock][half][Mp][512]
     const _Float16 *sums;   // [superblock][Mp][16]
     const float *unit;      // [Mp]: 1 / s of each row
-    const float *x;         // CONV: the activations themselves
-    int64_t x_stride;
-    int x_al16;
-    int64_t K;
     float *out;             // y, or the partials of segment 0
     int64_t out_stride;
     int64_t seg_stride;
@@ -531,14 +527,13 @@ __device__ __forceinline__ void gm_barrier() {
     __syncthreads();
 }
 
-template <int TYPE, int MT, bool CONV>
+template <int TYPE, int MT>
 __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     constexpr int BM = 32 * MT, NT = kGmNT;
     constexpr bool Q40 = TYPE == MI355X_TYPE_Q4_0;
     using Regs = typename RegsOf<TYPE>::T;
     __shared__ uint4 xh0[BM * kGmHalfBytes / 16], xh1[BM * kGmHalfBytes / 16];
     __shared__ uint4 ssum[2][BM * 2];
-    __shared__ float sscale[CONV ? BM : 1], sunit[CONV ? BM : 1];
     __shared__ uint2 tab[gm_table_entries(TYPE)];
 
     const int lane = threadIdx.x & 63;
@@ -773,24 +768,20 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
             dlast = 0.f;
         }
     };
-    // segment `seg` to out (CONV: added to the segments before it)
-    auto store = [&](int seg, auto unit) {
-        float *out = a.out + (CONV ? 0 : seg * a.seg_stride);
+    auto store = [&](int seg) {
+        float *out = a.out + seg * a.seg_stride;
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
                 const int m = m0 + 32 * i + 8 * (k >> 2) + 4 * h + (k & 3);
                 if (m >= a.M) continue;
-                const float u = unit(m);
+                const float u = a.unit[m];
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     const int64_t n = n0 + 32 * t + col;
                     if (n >= a.N) continue;
-                    float *p = out + m * a.out_stride + n;
-                    const float v = u * acc[t][i][k];
-                    if constexpr (CONV) *p = seg == 0 ? v : *p + v;
-                    else *p = v;
+                    out[m * a.out_stride + n] = u * acc[t][i][k];
                 }
             }
         }
@@ -801,88 +792,47 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     stage_table<TYPE>(a, tab);
     vlast = f32x16{};
 
-    if constexpr (CONV) {
-        const bool al16 = a.x_al16 != 0;
-        auto load = [&](int r, int b) {
-            const int64_t left = a.K - 256 * static_cast<int64_t>(b);
-            return load_x4(a.x + (m0 + r) * a.x_stride + 256 * static_cast<int64_t>(b), 4 * lane,
-                           static_cast<int>(left < 256 ? left : 256), al16);
-        };
-        for (int r = wave; r < BM && m0 + r < a.M; r += kGmWaves) {
-            float m = 0.f, u;
-            for (int b = 0; b < a.B; ++b) m = fmaxf(m, abs_max4(load(r, b)));
-            const float s = row_scale(wave_max(m), u);
-            if (lane == 0) {
-                sscale[r] = s;
-                sunit[r] = u;
-            }
-        }
-        for (int seg = 0; seg < a.nseg; ++seg) {
-            const int b0 = seg * a.per_seg, b1 = min(b0 + a.per_seg, a.B);
-            clear();
-            Regs r[2][NT];
-            for (int b = b0; b < b1; ++b) {
-                load_raw(r[0], b, 0, 0);
-                load_raw(r[1], b, 0, 1);
-                __syncthreads();  // scales written; the previous superblock's operands are read
-                for (int row = wave; row < BM && m0 + row < a.M; row += kGmWaves)
-                    store_superblock(convert_superblock(load(row, b), sscale[row]), row, lane,
-                                     reinterpret_cast<uint8_t *>(xh0) + kGmHalfBytes * row,
-                                     reinterpret_cast<uint8_t *>(xh1) + kGmHalfBytes * row,
-                                     reinterpret_cast<_Float16 *>(ssum[0]) + 16 * row);
-                __syncthreads();
-                decode_first(r);
-                half_step(r, xh0, H0{}, [&] { load_raw(r[0], b, 1, 0); });
-                load_raw(r[1], b, 1, 1);
-                half_step(r, xh1, H1{}, [&] {});
-                finish(r[1], 0);
-            }
-            flush();
-            store(seg, [&](int m) { return sunit[m - m0]; });
-        }
-    } else {
-        const int seg = blockIdx.y;
-        const int b0 = seg * a.per_seg, b1 = min(b0 + a.per_seg, a.B);
-        auto half_src = [&](int b, int half) {
-            return a.planes + (static_cast<int64_t>(2 * b + half) * a.Mp + m0) * kGmHalfBytes;
-        };
-        constexpr bool MINS = TYPE == MI355X_TYPE_Q4_K || TYPE == MI355X_TYPE_Q5_K;
-        // sums of superblock b (types with mins): threads 0 .. 2 BM - 1
-        auto load_sums = [&](int b, uint4 &s) {
-            if (MINS && threadIdx.x < 2 * BM)
-                s = reinterpret_cast<const uint4 *>(a.sums)[(static_cast<int64_t>(b) * a.Mp + m0) * 2 + threadIdx.x];
-        };
-        auto put_sums = [&](int par, const uint4 &s) {
-            if (MINS && threadIdx.x < 2 * BM) ssum[par][threadIdx.x] = s;
-        };
-        clear();
-        uint4 s = make_uint4(0, 0, 0, 0);
-        Regs r[2][NT];
-        copy_planes<BM>(half_src(b0, 0), xh0, wave, lane);
-        load_sums(b0, s);
-        load_raw(r[0], b0, 0, 0);
-        put_sums(b0 & 1, s);
+    const int seg = blockIdx.y;
+    const int b0 = seg * a.per_seg, b1 = min(b0 + a.per_seg, a.B);
+    auto half_src = [&](int b, int half) {
+        return a.planes + (static_cast<int64_t>(2 * b + half) * a.Mp + m0) * kGmHalfBytes;
+    };
+    constexpr bool MINS = TYPE == MI355X_TYPE_Q4_K || TYPE == MI355X_TYPE_Q5_K;
+    // sums of superblock b (types with mins): threads 0 .. 2 BM - 1
+    auto load_sums = [&](int b, uint4 &s) {
+        if (MINS && threadIdx.x < 2 * BM)
+            s = reinterpret_cast<const uint4 *>(a.sums)[(static_cast<int64_t>(b) * a.Mp + m0) * 2 + threadIdx.x];
+    };
+    auto put_sums = [&](int par, const uint4 &s) {
+        if (MINS && threadIdx.x < 2 * BM) ssum[par][threadIdx.x] = s;
+    };
+    clear();
+    uint4 s = make_uint4(0, 0, 0, 0);
+    Regs r[2][NT];
+    copy_planes<BM>(half_src(b0, 0), xh0, wave, lane);
+    load_sums(b0, s);
+    load_raw(r[0], b0, 0, 0);
+    put_sums(b0 & 1, s);
+    gm_barrier();
+    decode_first(r);
+    for (int b = b0; b < b1; ++b) {
+        const int bn = b + 1 < b1 ? b + 1 : b;  // the last superblock's look-ahead reads itself again
+        copy_planes<BM>(half_src(b, 1), xh1, wave, lane);
+        load_raw(r[1], b, 0, 1);
+        __builtin_amdgcn_sched_barrier(0);  // the loads go out before this half's work
+        half_step(r, xh0, H0{}, [&] { load_raw(r[0], b, 1, 0); });
         gm_barrier();
-        decode_first(r);
-        for (int b = b0; b < b1; ++b) {
-            const int bn = b + 1 < b1 ? b + 1 : b;  // the last superblock's look-ahead reads itself again
-            copy_planes<BM>(half_src(b, 1), xh1, wave, lane);
-            load_raw(r[1], b, 0, 1);
-            __builtin_amdgcn_sched_barrier(0);  // the loads go out before this half's work
-            half_step(r, xh0, H0{}, [&] { load_raw(r[0], b, 1, 0); });
-            gm_barrier();
-            copy_planes<BM>(half_src(bn, 0), xh0, wave, lane);
-            load_sums(bn, s);
-            load_raw(r[1], b, 1, 1);
-            __builtin_amdgcn_sched_barrier(0);
-            half_step(r, xh1, H1{}, [&] { load_raw(r[0], bn, 0, 0); });
-            finish(r[1], b & 1);
-            put_sums((b + 1) & 1, s);
-            gm_barrier();
-        }
-        flush();
-        store(seg, [&](int m) { return a.unit[m]; });
+        copy_planes<BM>(half_src(bn, 0), xh0, wave, lane);
+        load_sums(bn, s);
+        load_raw(r[1], b, 1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        half_step(r, xh1, H1{}, [&] { load_raw(r[0], bn, 0, 0); });
+        finish(r[1], b & 1);
+        put_sums((b + 1) & 1, s);
+        gm_barrier();
     }
+    flush();
+    store(seg);
 }
 
 // y = partial 0 + partial 1 + ..., in segment order
@@ -901,127 +851,115 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float *part, int
 typedef void (*gemm_fn)(GemmArgs);
 
 template <int TYPE>
-gemm_fn pick_gemm_type(int mt, bool conv) {
-    if (conv) return mt == 1 ? gemm_kernel<TYPE, 1, true> : gemm_kernel<TYPE, 2, true>;
-    return mt == 1 ? gemm_kernel<TYPE, 1, false> : gemm_kernel<TYPE, 2, false>;
+gemm_fn pick_gemm_type(int mt) {
+    return mt == 1 ? gemm_kernel<TYPE, 1> : gemm_kernel<TYPE, 2>;
 }
 
-gemm_fn pick_gemm(int type, int mt, bool conv) {
+gemm_fn pick_gemm(int type, int mt) {
     switch (type) {
-    case MI355X_TYPE_Q4_0: return pick_gemm_type<MI355X_TYPE_Q4_0>(mt, conv);
-    case MI355X_TYPE_Q3_K: return pick_gemm_type<MI355X_TYPE_Q3_K>(mt, conv);
-    case MI355X_TYPE_Q4_K: return pick_gemm_type<MI355X_TYPE_Q4_K>(mt, conv);
-    case MI355X_TYPE_Q5_K: return pick_gemm_type<MI355X_TYPE_Q5_K>(mt, conv);
-    case MI355X_TYPE_Q6_K: return pick_gemm_type<MI355X_TYPE_Q6_K>(mt, conv);
-    case MI355X_TYPE_IQ4_XS: return pick_gemm_type<MI355X_TYPE_IQ4_XS>(mt, conv);
-    case MI355X_TYPE_IQ3_S: return pick_gemm_type<MI355X_TYPE_IQ3_S>(mt, conv);
-    case MI355X_TYPE_IQ3_XXS: return pick_gemm_type<MI355X_TYPE_IQ3_XXS>(mt, conv);
-    case MI355X_TYPE_IQ2_S: return pick_gemm_type<MI355X_TYPE_IQ2_S>(mt, conv);
+    case MI355X_TYPE_Q4_0: return pick_gemm_type<MI355X_TYPE_Q4_0>(mt);
+    case MI355X_TYPE_Q3_K: return pick_gemm_type<MI355X_TYPE_Q3_K>(mt);
+    case MI355X_TYPE_Q4_K: return pick_gemm_type<MI355X_TYPE_Q4_K>(mt);
+    case MI355X_TYPE_Q5_K: return pick_gemm_type<MI355X_TYPE_Q5_K>(mt);
+    case MI355X_TYPE_Q6_K: return pick_gemm_type<MI355X_TYPE_Q6_K>(mt);
+    case MI355X_TYPE_IQ4_XS: return pick_gemm_type<MI355X_TYPE_IQ4_XS>(mt);
+    case MI355X_TYPE_IQ3_S: return pick_gemm_type<MI355X_TYPE_IQ3_S>(mt);
+    case MI355X_TYPE_IQ3_XXS: return pick_gemm_type<MI355X_TYPE_IQ3_XXS>(mt);
+    case MI355X_TYPE_IQ2_S: return pick_gemm_type<MI355X_TYPE_IQ2_S>(mt);
     default: return nullptr;
     }
 }
 
-constexpr size_t kGmPartialMax = size_t(64) << 20;
-
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+
+// Rows of activation tiles for M activations, and what their planes, sums and
+// units take of the workspace.
+int tile_rows(int M) { return M <= 32 ? 32 : (M + 63) / 64 * 64; }
+size_t planes_bytes(int64_t B, int Mp) { return static_cast<size_t>(B) * 2 * Mp * kGmHalfBytes; }
+size_t sums_bytes(int64_t B, int Mp) { return align256(static_cast<size_t>(B) * Mp * 32); }
+size_t staged_bytes(int64_t B, int Mp) {
+    return planes_bytes(B, Mp) + sums_bytes(B, Mp) + align256(static_cast<size_t>(Mp) * 4);
+}
 
 }  // namespace
 
-// From how many activations the matrix cores take a call: for the K/IQ types,
-// whose alternative is one GEMV each (7-12 us at the FFN shapes against 40 us
-// for up to 64 here), from 4; for Q4_0 from 16, past two passes of the 8-row
-// kernels.
+// From how many activations the matrix cores take a call.  For the K/IQ types,
+// whose alternative is one GEMV each (us, that first: 34 / 23 at Q4_K 64x16384 M
+// = 4, 35 / 25 at 3001x2816), from 4, but from 5 for codebook matrices of few
+// rows (IQ3_S 1024x4096: 16 / 19 at M = 4, 20 / 19 at 5).  For Q4_0 past two
+// passes of the 8-row kernels (M = 24: 26 / 21 at 256x4096, 51 / 28 at
+// 4096x8192); with 2^25 weights and more also most of two passes (29 / 24 at
+// 4096x8192 M = 12, 34 / 25 at M = 16; smaller ones not: 18 / 20 at 256x4096).
 bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) {
     if (ctx->kernel_variant != MI355X_VARIANT_AUTO && ctx->kernel_variant != MI355X_VARIANT_DIGITS) return false;
-    if (a.x_bf16 || a.N <= 0 || a.K <= 0) return false;
+    if (a.x_bf16 || a.N <= 0 || a.K <= 0 || !ctx->gemm_buf) return false;
     // 32-bit offsets into the 64 rows of a wavefront
     const int64_t row_bytes = a.type == MI355X_TYPE_Q4_0 ? a.K / 32 * 18 : a.K / 256 * kq_layout(a.type).block_bytes;
     if (row_bytes <= 0 || row_bytes >= (int64_t(1) << 31) / 64 || a.N >= (int64_t(1) << 31)) return false;
+    if (staged_bytes((a.K + 255) / 256, 32) > kGemmWorkspace) return false;
     if (a.type == MI355X_TYPE_Q4_0) {
         // dword-aligned loads of code groups
         if (reinterpret_cast<uintptr_t>(a.W) % 4 != 0 || row_bytes % 4 != 0) return false;
-        return M >= 16;
+        return M >= 17 || (M >= 12 && a.N * a.K >= (int64_t(1) << 25));
     }
     // codes times scales exact in f16
     if ((a.type == MI355X_TYPE_IQ3_XXS || a.type == MI355X_TYPE_IQ2_S) &&
         (a.type == MI355X_TYPE_IQ3_XXS ? ctx->iq3xxs_max : ctx->iq2s_max) > 66)
         return false;
-    return M >= 4;
+    return M >= (a.N < 4096 && !kq_digit_rows(ctx, a.type, a.N, a.K) ? 5 : 4);
 }
 
-int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int64_t M_total,
-                        bool noalloc) {
+// The workspace belongs to the context from its creation to its end and never
+// moves, so no call allocates and a captured call stays valid; the context's
+// lock keeps the launches that share it together on its stream.  Activations
+// that it cannot hold at once go in several passes.
+int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int64_t M_total) {
     const bool q40 = a.type == MI355X_TYPE_Q4_0;
-    const int64_t row_bytes = q40 ? a.K / 32 * 18 : a.K / 256 * kq_layout(a.type).block_bytes;
     GemmArgs g{};
     g.W = a.W;
     g.N = a.N;
-    g.K = a.K;
-    g.row_bytes = row_bytes;
+    g.row_bytes = q40 ? a.K / 32 * 18 : a.K / 256 * kq_layout(a.type).block_bytes;
     g.B = static_cast<int>((a.K + 255) / 256);
     g.blocks = static_cast<int>(a.K / 32);
-    g.x_stride = x_stride;
-    g.x_al16 = reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && x_stride % 4 == 0 ? 1 : 0;
+    const int x_al16 = reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && x_stride % 4 == 0 ? 1 : 0;
     if (a.type == MI355X_TYPE_IQ3_XXS) g.grid = static_cast<const uint32_t *>(ctx->iq3xxs_grid);
     if (a.type == MI355X_TYPE_IQ2_S) g.grid = static_cast<const uint32_t *>(ctx->iq2s_grid);
     if ((a.type == MI355X_TYPE_IQ3_XXS || a.type == MI355X_TYPE_IQ2_S) && !g.grid)
         return set_error(MI355X_EUNSUPPORTED, "grid table not installed for this IQ type");
     g.ntiles = static_cast<int>((a.N + kGmCols - 1) / kGmCols);
-    std::unique_lock<std::mutex> lk(ctx->mu, std::defer_lock);
-    if (!noalloc) lk.lock();
-    for (int64_t mb = 0; mb < M_total; mb += kGmMaxRows) {
-        const int M = static_cast<int>(std::min<int64_t>(kGmMaxRows, M_total - mb));
+    std::lock_guard<std::mutex> lk(ctx->mu);
+    for (int64_t mb = 0; mb < M_total; mb += g.M) {
+        int M = static_cast<int>(std::min<int64_t>(kGmMaxRows, M_total - mb));
+        while (M > 32 && staged_bytes(g.B, tile_rows(M)) > kGemmWorkspace) M = std::max(32, (M / 2 + 31) / 32 * 32);
         const int mt = M <= 32 ? 1 : 2;
         g.M = M;
-        g.mtiles = (M + 32 * mt - 1) / (32 * mt);
-        g.Mp = g.mtiles * 32 * mt;
-        g.x = static_cast<const float *>(a.x) + mb * x_stride;
+        g.Mp = tile_rows(M);
+        g.mtiles = g.Mp / (32 * mt);
         float *y = a.y + mb * y_stride;
         const int64_t tiles = static_cast<int64_t>(g.ntiles) * g.mtiles;
+        const size_t staged = staged_bytes(g.B, g.Mp);
         // segments of K: enough workgroups for two per CU, at least two
-        // superblocks each, partials within kGmPartialMax
+        // superblocks each, partials within the rest of the workspace
         int64_t seg = std::max<int64_t>(1, 2 * ctx->num_cus / tiles);
         seg = std::min<int64_t>(seg, std::max(1, g.B / 2));
-        seg = std::min<int64_t>(seg, std::max<int64_t>(1, static_cast<int64_t>(kGmPartialMax / (4 * M * a.N))));
+        seg = std::min<int64_t>(seg, std::max<int64_t>(1, static_cast<int64_t>(kGemmWorkspace - staged) / (4 * M * a.N)));
         g.per_seg = static_cast<int>((g.B + seg - 1) / seg);
         g.nseg = (g.B + g.per_seg - 1) / g.per_seg;
         const unsigned grid_x = static_cast<unsigned>((g.ntiles + 7) / 8 * 8 * g.mtiles);
-        const gemm_fn k = pick_gemm(a.type, mt, noalloc);
-        if (noalloc) {
-            // planes converted by each workgroup, segments one after another:
-            // the same sums in the same order, no buffer
-            g.out = y;
-            g.out_stride = y_stride;
-            hipLaunchKernelGGL(k, dim3(grid_x), dim3(kGmThreads), 0, ctx->stream, g);
-            MI355X_HIP(hipGetLastError());
-            continue;
-        }
-        const size_t planes = static_cast<size_t>(g.B) * 2 * g.Mp * kGmHalfBytes;
-        const size_t sums = static_cast<size_t>(g.B) * g.Mp * 32;
-        const size_t units = align256(static_cast<size_t>(g.Mp) * 4);
-        const size_t part = g.nseg > 1 ? static_cast<size_t>(g.nseg) * M * a.N * 4 : 0;
-        const size_t need = planes + align256(sums) + units + part;
-        if (ctx->gemm_bytes < need) {
-            const int rc = free_device(ctx, ctx->gemm_buf);
-            if (rc) return rc;
-            ctx->gemm_buf = nullptr;
-            ctx->gemm_bytes = 0;
-            MI355X_HIP(hipMalloc(&ctx->gemm_buf, need));
-            ctx->gemm_bytes = need;
-        }
         uint8_t *p = static_cast<uint8_t *>(ctx->gemm_buf);
         g.planes = p;
-        g.sums = reinterpret_cast<const _Float16 *>(p + planes);
-        g.unit = reinterpret_cast<const float *>(p + planes + align256(sums));
-        float *partial = reinterpret_cast<float *>(p + planes + align256(sums) + units);
+        g.sums = reinterpret_cast<const _Float16 *>(p + planes_bytes(g.B, g.Mp));
+        g.unit = reinterpret_cast<const float *>(p + planes_bytes(g.B, g.Mp) + sums_bytes(g.B, g.Mp));
+        float *partial = reinterpret_cast<float *>(p + staged);
         g.out = g.nseg > 1 ? partial : y;
         g.out_stride = g.nseg > 1 ? a.N : y_stride;
         g.seg_stride = static_cast<int64_t>(M) * a.N;
-        hipLaunchKernelGGL(gemm_planes_kernel, dim3(static_cast<unsigned>(M)), dim3(kPlThreads), 0, ctx->stream, g.x,
-                           x_stride, a.K, g.x_al16, g.Mp, g.B, p, const_cast<_Float16 *>(g.sums),
-                           const_cast<float *>(g.unit));
+        hipLaunchKernelGGL(gemm_planes_kernel, dim3(static_cast<unsigned>(M)), dim3(kPlThreads), 0, ctx->stream,
+                           static_cast<const float *>(a.x) + mb * x_stride, x_stride, a.K, x_al16, g.Mp, g.B, p,
+                           const_cast<_Float16 *>(g.sums), const_cast<float *>(g.unit));
         MI355X_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k, dim3(grid_x, static_cast<unsigned>(g.nseg)), dim3(kGmThreads), 0, ctx->stream, g);
+        hipLaunchKernelGGL(pick_gemm(a.type, mt), dim3(grid_x, static_cast<unsigned>(g.nseg)), dim3(kGmThreads), 0,
+                           ctx->stream, g);
         MI355X_HIP(hipGetLastError());
         if (g.nseg > 1) {
             hipLaunchKernelGGL(gemm_reduce_kernel, dim3(static_cast<unsigned>((a.N + 255) / 256), std::min(M, 64)),

@@ -28,10 +28,10 @@ struct mi355x_ctx {
     // demand, freed with the context)
     void *mbtiles = nullptr;
     size_t mbtiles_bytes = 0;
-    // activation planes and K-segment partials of a matrix-core batched call
-    // (grown on demand, freed with the context)
+    // activation planes and K-segment partials of a matrix-core batched call:
+    // kGemmWorkspace bytes from the context's creation to its end, never moved
+    // (null if the device had no room: such calls take the other forms)
     void *gemm_buf = nullptr;
-    size_t gemm_bytes = 0;
     // device address of the library's static scratch on this device
     // (allocation-free entry point)
     void *scratch = nullptr;
@@ -125,11 +125,10 @@ int launch_gemv_q4_0_mb(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
 int resolve_scratch(int device, void **out);
 size_t scratch_bytes();
 // Matrix-core form of a batched call (any weight type): whether it takes M
-// activation rows of `a`, and its launches.  noalloc: no context buffer; the
-// same outputs bit for bit.
+// activation rows of `a`, and its launches.
+constexpr size_t kGemmWorkspace = size_t(64) << 20;
 bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M);
-int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int64_t M,
-                        bool noalloc);
+int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int64_t M);
 // Several Q4_0 matrices that share the activation row x as one launch of
 // the pipelined form (*launched = false where that form does not apply: the
 // caller launches each matrix on its own).

@@ -407,6 +407,11 @@ int mi355x_ctx_create(int device, mi355x_ctx **out) {
         mi355x_ctx_destroy(ctx);
         return set_error(rc, msg);
     }
+    // batched calls do without it if the device has no room
+    if (hipMalloc(&ctx->gemm_buf, kGemmWorkspace) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->gemm_buf = nullptr;
+    }
     *out = ctx;
     return MI355X_OK;
 }
@@ -938,7 +943,7 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
         }
         GemvArgs a{type, static_cast<const uint8_t *>(W), N, K, x, false, y};
         if (kq_mx_takes(ctx, a, M)) return launch_gemv_kq_mx(ctx, a, x_stride, y_stride, static_cast<int>(M));
-        if (gemm_batched_supports(ctx, a, M)) return launch_gemm_batched(ctx, a, x_stride, y_stride, M, noalloc);
+        if (gemm_batched_supports(ctx, a, M)) return launch_gemm_batched(ctx, a, x_stride, y_stride, M);
     }
     // Q4_0 digit-plane arithmetic: up to q4_0_mb_capacity() activations per
     // launch of the batched form (weights read once per launch)
