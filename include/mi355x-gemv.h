@@ -295,10 +295,12 @@ MI355X_API int mi355x_gemv_bf16(mi355x_ctx *ctx, int type, const void *W, int64_
  * IQ2_S with grids of magnitudes up to 66).  A few activations (2 to 8, as
  * many as fit the LDS) of the other types run in one launch with the one-row
  * kernels' digit arithmetic on the integer matrix cores, where those kernels
- * use it and K <= 16384.  Fewer Q4_0 activations with the
- * digit-plane arithmetic, rows a multiple of 256 values and 16-byte aligned
- * weights: up to 8 per pass (one staging launch into a context buffer, one
- * batched launch).  Other cases:
+ * use it and K <= 16384.  Fewer Q4_0 activations, rows a multiple of 256
+ * values and 16-byte aligned weights: up to 8 per pass, on the matrix cores (one
+ * launch, activations as two f16 planes) where that is the faster form (most
+ * sizes from 5 activations, short rows from 2), else with the digit-plane
+ * arithmetic (one staging launch into a context buffer, one batched launch; or
+ * one launch).  Other cases:
  * M sequential GEMVs.  Calls on one context serialise on its lock while
  * they enqueue. */
 MI355X_API int mi355x_gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,

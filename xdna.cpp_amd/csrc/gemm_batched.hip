@@ -887,9 +887,9 @@ size_t staged_bytes(int64_t B, int Mp) {
 // whose alternative is one GEMV each (us, that first: 34 / 23 at Q4_K 64x16384 M
 // = 4, 35 / 25 at 3001x2816), from 4, but from 5 for codebook matrices of few
 // rows (IQ3_S 1024x4096: 16 / 19 at M = 4, 20 / 19 at 5).  For Q4_0 past two
-// passes of the 8-row kernels (M = 24: 26 / 21 at 256x4096, 51 / 28 at
-// 4096x8192); with 2^25 weights and more also most of two passes (29 / 24 at
-// 4096x8192 M = 12, 34 / 25 at M = 16; smaller ones not: 18 / 20 at 256x4096).
+// passes of the 8-row kernels; with 2^25 weights of long rows also most of two
+// passes (31 / 24 at 4096x8192 M = 12, 40 / 36 at 8192x8192 M = 16; but 16 / 20
+// at 256x4096, 97 / 122 at 151936x2048).
 bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) {
     if (ctx->kernel_variant != MI355X_VARIANT_AUTO && ctx->kernel_variant != MI355X_VARIANT_DIGITS) return false;
     if (a.x_bf16 || a.N <= 0 || a.K <= 0 || !ctx->gemm_buf) return false;
@@ -900,7 +900,7 @@ bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) 
     if (a.type == MI355X_TYPE_Q4_0) {
         // dword-aligned loads of code groups
         if (reinterpret_cast<uintptr_t>(a.W) % 4 != 0 || row_bytes % 4 != 0) return false;
-        return M >= 17 || (M >= 12 && a.N * a.K >= (int64_t(1) << 25));
+        return M >= 17 || (M >= 12 && a.K >= 4096 && a.N * a.K >= (int64_t(1) << 25));
     }
     // codes times scales exact in f16
     if ((a.type == MI355X_TYPE_IQ3_XXS || a.type == MI355X_TYPE_IQ2_S) &&

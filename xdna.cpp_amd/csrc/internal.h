@@ -120,6 +120,10 @@ int q4_0_mb_capacity(const mi355x_ctx *ctx, const GemvArgs &a);
 // null for the context's own tile buffer (grown with hipMalloc on demand).
 int launch_gemv_q4_0_mb(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int M,
                         void *fixed_tiles);
+// The same rows on the matrix cores, without a buffer, and whether that form is
+// the faster one for a call of M activations.
+bool q4_0_mx_takes(const GemvArgs &a, int64_t M);
+int launch_gemv_q4_0_mx(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int M);
 // Device address of the static scratch on `device` (the device must be
 // current); resolved once per device with hipGetSymbolAddress.
 int resolve_scratch(int device, void **out);

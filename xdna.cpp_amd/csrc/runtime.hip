@@ -945,8 +945,8 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
         if (kq_mx_takes(ctx, a, M)) return launch_gemv_kq_mx(ctx, a, x_stride, y_stride, static_cast<int>(M));
         if (gemm_batched_supports(ctx, a, M)) return launch_gemm_batched(ctx, a, x_stride, y_stride, M);
     }
-    // Q4_0 digit-plane arithmetic: up to q4_0_mb_capacity() activations per
-    // launch of the batched form (weights read once per launch)
+    // Q4_0: up to q4_0_mb_capacity() activations per launch (weights read once
+    // per launch), on the matrix cores or in digit-plane arithmetic
     if (ctx && type == MI355X_TYPE_Q4_0 && M >= 2 && N > 0 && W && x && y &&
         (ctx->kernel_variant == MI355X_VARIANT_AUTO || ctx->kernel_variant == MI355X_VARIANT_DIGITS)) {
         uint64_t total = 0;
@@ -956,12 +956,14 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
         const int cap = q4_0_mb_capacity(ctx, a);
         if (cap >= 2) {
             DeviceGuard dg(ctx->device);
+            const bool mx = q4_0_mx_takes(a, M);
             for (int64_t m0 = 0; m0 < M;) {
                 const int chunk = static_cast<int>(std::min<int64_t>(cap, M - m0));
                 GemvArgs c{type, static_cast<const uint8_t *>(W), N, K, x + m0 * x_stride, false, y + m0 * y_stride};
                 // a one-activation remainder also runs in this form, so every
                 // output of the call has the same arithmetic
-                rc = launch_gemv_q4_0_mb(ctx, c, x_stride, y_stride, chunk, noalloc ? ctx->scratch : nullptr);
+                rc = mx ? launch_gemv_q4_0_mx(ctx, c, x_stride, y_stride, chunk)
+                        : launch_gemv_q4_0_mb(ctx, c, x_stride, y_stride, chunk, noalloc ? ctx->scratch : nullptr);
                 if (rc) return rc;
                 m0 += chunk;
             }
