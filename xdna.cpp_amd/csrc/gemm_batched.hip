@@ -888,7 +888,7 @@ size_t staged_bytes(int64_t B, int Mp) {
 // = 4, 35 / 25 at 3001x2816), from 4, but from 5 for codebook matrices of few
 // rows (IQ3_S 1024x4096: 16 / 19 at M = 4, 20 / 19 at 5).  For Q4_0 past two
 // passes of the 8-row kernels; with 2^25 weights of long rows also most of two
-// passes (31 / 24 at 4096x8192 M = 12, 40 / 36 at 8192x8192 M = 16; but 16 / 20
+// passes (30 / 24 at 4096x8192 M = 12, 39 / 36 at 8192x8192 M = 16; but 16 / 20
 // at 256x4096, 97 / 122 at 151936x2048).
 bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) {
     if (ctx->kernel_variant != MI355X_VARIANT_AUTO && ctx->kernel_variant != MI355X_VARIANT_DIGITS) return false;

@@ -19,17 +19,17 @@
 // row n; a 4 x 4 exchange between the lane groups (permlane swaps) gives every
 // lane dword g of all four blocks, the 8 codes of its MFMA operand.  The
 // wavefront's activations stay in registers (4 per block), read from the
-// caller once per workgroup: the lanes of the two planes of a row each load
-// every other block and exchange the plane that the other one needs.  A quad's
+// caller once per workgroup: the lanes of the two planes of a row each load half
+// of every block and exchange the plane that the other one needs.  A quad's
 // registers are reloaded with the next tile's right after its decode, so QN
 // quads per wavefront stay in flight; tile sums meet in LDS.  Rows of more than
 // 8192 values go in two launches, the second adding to y.
 //
-// What bounds it.  VALU issue: about 85 instructions per quad and tile and 100
+// What bounds it.  VALU issue: about 85 instructions per quad and tile and 78
 // per quad to stage the activations, which every workgroup does for itself, so
 // long rows with few tiles per workgroup spend most of their time staging.
-// us per call on MI355X, dot-unit forms -> here: M = 8 8192x8192 25.9 -> 20.0,
-// 4096x4096 11.9 -> 8.3, 17408x5120 42.9 -> 20.1, 151936x2048 73.7 -> 48.3.
+// us per call on MI355X, dot-unit forms -> here: M = 8 8192x8192 25.9 -> 19.3,
+// 4096x4096 11.9 -> 8.2, 17408x5120 42.9 -> 19.7, 151936x2048 73.7 -> 49.
 #include "internal.h"
 #include "kq_device.h"
 #include "q4_0_layout.h"
@@ -106,13 +106,14 @@ __device__ __forceinline__ float4 qx_load4(const float *p) {
     __builtin_memcpy(&f, p, sizeof f);
     return f;
 }
-// x s rounded to f16, and what that leaves (x s is exact: one rounding each)
-__device__ __forceinline__ f16x2 qx_hi(float x0, float x1, float s) {
-    return f16x2{static_cast<_Float16>(x0 * s), static_cast<_Float16>(x1 * s)};
+// w rounded to f16, and what that leaves
+__device__ __forceinline__ f16x2 qx_hi(float w0, float w1) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    return __builtin_convertvector((f32x2{w0, w1}), f16x2);
 }
-__device__ __forceinline__ f16x2 qx_lo(float x0, float x1, float s, f16x2 h) {
-    return f16x2{static_cast<_Float16>(fmaf(x0, s, -static_cast<float>(h[0]))),
-                 static_cast<_Float16>(fmaf(x1, s, -static_cast<float>(h[1])))};
+__device__ __forceinline__ f16x2 qx_lo(float w0, float w1, f16x2 h) {
+    return f16x2{static_cast<_Float16>(w0 - static_cast<float>(h[0])),
+                 static_cast<_Float16>(w1 - static_cast<float>(h[1]))};
 }
 // `own` in the lanes of one plane (banks of 4 lanes of a 16-lane row), the
 // other plane's lanes of `other` in the rest: row_ror:8
@@ -121,10 +122,6 @@ __device__ __forceinline__ uint32_t qx_from(f16x2 own, f16x2 other) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(__builtin_bit_cast(int, own),
                                                              __builtin_bit_cast(int, other), 0x128, 0xF, BANKS, false));
 }
-__device__ __forceinline__ float qx_abs4(const float4 &f) {
-    return fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w)));
-}
-
 template <int QN>
 __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     __shared__ f32x4 part[2][kQxWaves][64];
@@ -135,19 +132,17 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     const int m = col & 7, plane = col >> 3;
     const int qw = a.q0 + wave * QN;  // first quad of the wavefront
 
-    // 1. its activations: of quad i, blocks plane and 2 + plane
+    // 1. its activations: of every block, values 16 plane + 4 g + (0..3), so that
+    // the lanes of a row read whole cache lines
     // (rows past M and quads past the launch's repeat the last: their products
     // are not stored, or are with zero weights)
-    float4 f[QN][2][2];
-    const float *xr = a.x + min(m, a.M - 1) * a.x_stride + 4 * g + 32 * plane;
+    float4 f[QN][4];
+    const float *xr = a.x + min(m, a.M - 1) * a.x_stride + 4 * g + 16 * plane;
 #pragma unroll
     for (int i = 0; i < QN; ++i) {
         const float *p = xr + 128 * static_cast<int64_t>(min(qw + i, a.q1 - 1));
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            f[i][e][0] = qx_load4(p + 64 * e);
-            f[i][e][1] = qx_load4(p + 64 * e + 16);
-        }
+        for (int e = 0; e < 4; ++e) f[i][e] = qx_load4(p + 32 * e);
     }
 
     // 2. the first tile's weights
@@ -177,11 +172,15 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     __builtin_amdgcn_sched_barrier(0);
 
     // 3. the activations' operands
-    float mx = 0.f;
+    float mxe[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < QN; ++i)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) mx = fmaxf(mx, qx_abs4(f[i][k >> 1][k & 1]));
+        for (int e = 0; e < 4; ++e) {
+            mxe[e] = fmaxf(fmaxf(mxe[e], fabsf(f[i][e].x)), fabsf(f[i][e].y));
+            mxe[e] = fmaxf(fmaxf(mxe[e], fabsf(f[i][e].z)), fabsf(f[i][e].w));
+        }
+    float mx = fmaxf(fmaxf(mxe[0], mxe[1]), fmaxf(mxe[2], mxe[3]));
     mx = fmaxf(mx, dpp_mov<0x128>(mx));  // row_ror:8, the row's other plane
     mx = fmaxf(mx, __shfl_xor(mx, 16));
     mx = fmaxf(mx, __shfl_xor(mx, 32));
@@ -193,20 +192,14 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
 #pragma unroll
     for (int i = 0; i < QN; ++i) {
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            u32x4 first, second;
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                const float4 &v = f[i][e][k];
-                const f16x2 h0 = qx_hi(v.x, v.z, s), h1 = qx_hi(v.y, v.w, s);
-                const f16x2 l0 = qx_lo(v.x, v.z, s, h0), l1 = qx_lo(v.y, v.w, s, h1);
-                first[2 * k] = qx_from<0xC>(h0, l0);
-                first[2 * k + 1] = qx_from<0xC>(h1, l1);
-                second[2 * k] = qx_from<0x3>(l0, h0);
-                second[2 * k + 1] = qx_from<0x3>(l1, h1);
-            }
-            x[i][2 * e] = __builtin_bit_cast(f16x8, first);
-            x[i][2 * e + 1] = __builtin_bit_cast(f16x8, second);
+        for (int e = 0; e < 4; ++e) {
+            const float4 &v = f[i][e];
+            const float w[4] = {v.x * s, v.y * s, v.z * s, v.w * s};
+            const f16x2 h0 = qx_hi(w[0], w[2]), h1 = qx_hi(w[1], w[3]);
+            const f16x2 l0 = qx_lo(w[0], w[2], h0), l1 = qx_lo(w[1], w[3], h1);
+            // values 4 g + (0..3) from the lane of plane 0, 16 + 4 g + (0..3) from plane 1's
+            const u32x4 o{qx_from<0xC>(h0, l0), qx_from<0xC>(h1, l1), qx_from<0x3>(l0, h0), qx_from<0x3>(l1, h1)};
+            x[i][e] = __builtin_bit_cast(f16x8, o);
         }
     }
     // result row 4 g + k of this wavefront is activation (4 g + k) & 7
@@ -271,12 +264,12 @@ qx_fn pick_qx(int qn) {
 
 // Where this form is faster than the dot-unit ones (us, those first).  From 5
 // activations, which cost those as much as 8: rows of up to 4096 values (M = 8
-// 256x512 8.0 / 4.5, 1024x4096 9.3 / 8.3), longer ones where enough tiles share
-// the staging (M = 8 4096x8192 17.3 / 15.6, 17408x14336 82 / 67; but 1024x8192
+// 256x512 8.0 / 4.6, 1024x4096 9.3 / 8.2), longer ones where enough tiles share
+// the staging (M = 8 4096x8192 17.3 / 15.1, 17408x14336 82 / 66; but 1024x8192
 // 9.7 / 15.6, 4096x14336 25.5 / 29.9).  Up to 4: where those need a staging
 // launch (the pipelined batched form does not: M = 2 4096x4096 5.2 / 7.1) and
-// rows are short (M = 4 1024x3072 7.6 / 5.9, M = 2 4096x5120 10.3 / 8.6, M = 4
-// 4096x6144 13.3 / 10.6; but M = 2 4096x7168 9.8 / 11.2, M = 4 1024x5120 7.3 /
+// rows are short (M = 4 1024x2560 7.4 / 5.7, M = 2 4096x5120 10.3 / 7.7, M = 4
+// 4096x6144 13.3 / 9.8; but M = 2 4096x7168 9.8 / 11.2, M = 4 1024x5120 7.3 /
 // 8.8).
 bool q4_0_mx_takes(const GemvArgs &a, int64_t M) {
     if (M >= 5) return a.K <= 4096 || a.N >= (a.K <= 8192 ? 4096 : 16384);
