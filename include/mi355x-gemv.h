@@ -284,7 +284,7 @@ MI355X_API int mi355x_gemv_bf16(mi355x_ctx *ctx, int type, const void *W, int64_
 /* M activation rows at once (row m at x + m*x_stride floats, output at
  * y + m*y_stride floats); the M-row case the reference admits for weights in
  * its own buffer type and computes as M sequential GEMVs
- * (src/ggml-xdna.cpp:110-112, 287-296).  In the variants AUTO and DIGITS many
+ * (src/ggml-xdna.cpp:110-112, 287-296).  In the variant AUTO many
  * activations (for Q4_0 with an even number of blocks per row M >= 17, from 2^25
  * weights M >= 12; for the other types M >= 4, or 5 where the one-row kernels
  * sum a codebook type in f32) run on the matrix cores, up to 512 per pass over
@@ -295,14 +295,16 @@ MI355X_API int mi355x_gemv_bf16(mi355x_ctx *ctx, int type, const void *W, int64_
  * IQ2_S with grids of magnitudes up to 66).  A few activations (2 to 8, as
  * many as fit the LDS) of the other types run in one launch with the one-row
  * kernels' digit arithmetic on the integer matrix cores, where those kernels
- * use it and K <= 16384.  Fewer Q4_0 activations, rows a multiple of 256
- * values and 16-byte aligned weights: up to 8 per pass, on the matrix cores (one
- * launch, activations as two f16 planes) where that is the faster form (most
- * sizes from 5 activations, short rows from 2), else with the digit-plane
- * arithmetic (one staging launch into a context buffer, one batched launch; or
- * one launch).  Other cases:
- * M sequential GEMVs.  Calls on one context serialise on its lock while
- * they enqueue. */
+ * use it (AUTO and DIGITS) and K <= 16384.  Fewer Q4_0 activations, rows a
+ * multiple of 256 values and 16-byte aligned weights: up to 8 per pass, on the
+ * matrix cores (AUTO; one launch, activations as two f16 planes) where that is
+ * the faster form (most sizes from 5 activations, short rows from 2), else, and
+ * always in DIGITS, with the digit-plane arithmetic (one staging launch into a
+ * context buffer, one batched launch; or one launch).  Other cases: M
+ * sequential GEMVs; so are calls on a context whose form, rows, wavefronts
+ * (Q4_0) or prefetch option is set, but for the digit-plane Q4_0 forms, and
+ * calls of many activations with MI355X_OPT_GRID set.  Calls on one context
+ * serialise on its lock while they enqueue. */
 MI355X_API int mi355x_gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
                                    const float *x, int64_t x_stride, float *y, int64_t y_stride,
                                    int64_t M);

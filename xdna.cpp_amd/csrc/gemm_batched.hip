@@ -889,9 +889,11 @@ size_t staged_bytes(int64_t B, int Mp) {
 // rows (IQ3_S 1024x4096: 16 / 19 at M = 4, 20 / 19 at 5).  For Q4_0 past two
 // passes of the 8-row kernels; with 2^25 weights of long rows also most of two
 // passes (30 / 24 at 4096x8192 M = 12, 39 / 36 at 8192x8192 M = 16; but 16 / 20
-// at 256x4096, 97 / 122 at 151936x2048).
+// at 256x4096, 97 / 122 at 151936x2048).  Only where the caller leaves arithmetic
+// and form to the library: MI355X_VARIANT_DIGITS promises fixed point, and the
+// kernels here know no form options and no cap on the workgroups.
 bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) {
-    if (ctx->kernel_variant != MI355X_VARIANT_AUTO && ctx->kernel_variant != MI355X_VARIANT_DIGITS) return false;
+    if (ctx->kernel_variant != MI355X_VARIANT_AUTO || !form_is_auto(ctx, a.type) || ctx->grid_override != 0) return false;
     if (a.x_bf16 || a.N <= 0 || a.K <= 0 || !ctx->gemm_buf) return false;
     // 32-bit offsets into the 64 rows of a wavefront
     const int64_t row_bytes = a.type == MI355X_TYPE_Q4_0 ? a.K / 32 * 18 : a.K / 256 * kq_layout(a.type).block_bytes;

@@ -759,6 +759,7 @@ mx_fn pick_mx(int type, int nu, int mb) {
 //          more than 6 activations of 4096 values one workgroup fits a CU
 bool kq_mx_takes(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) {
     if (a.type == MI355X_TYPE_Q4_0 || a.x_bf16 || M < 2 || M > kMxMaxAct || a.N <= 0 || a.N >= (int64_t(1) << 31)) return false;
+    if (!form_is_auto(ctx, a.type)) return false;
     const int64_t B = a.K / 256;
     if (B < 1 || B > kMxMaxBlocks || !kq_digit_rows(ctx, a.type, a.N, a.K)) return false;
     const size_t fixed = kMxRowSlots * kMxWaves * kMxRows * sizeof(float) + dg_table_words(a.type) * 4u + 256;

@@ -2313,12 +2313,12 @@ namespace mi355x {
 typedef void (*mb_kernel_t)(const uint8_t *, const uint4 *, float *, int64_t, int, int, int64_t, int);
 typedef void (*plm_kernel_t)(const uint8_t *, const float *, int64_t, int, float *, int64_t, int, int, int);
 
-// the pipelined batched variant: NBL full columns with NBL x MB <= 8 and MB <= 4
-// (more activations of such rows run on the matrix cores)
+// the pipelined batched variant: NBL full columns with NBL x MB <= 8
 plm_kernel_t pick_plm(int nbl, int mb) {
     switch (nbl * 16 + mb) {
     case 16 + 2: return gemv_q4_0_plm_kernel<1, 2>;
     case 16 + 4: return gemv_q4_0_plm_kernel<1, 4>;
+    case 16 + 8: return gemv_q4_0_plm_kernel<1, 8>;
     case 32 + 2: return gemv_q4_0_plm_kernel<2, 2>;
     case 32 + 4: return gemv_q4_0_plm_kernel<2, 4>;
     case 48 + 2: return gemv_q4_0_plm_kernel<3, 2>;
@@ -2336,9 +2336,10 @@ mb_kernel_t pick_mb_m(int mb) {
     }
 }
 
-// rows of up to two columns run in the pipelined form or on the matrix cores
 mb_kernel_t pick_mb(int nbl, int mb) {
     switch (nbl) {
+    case 1: return pick_mb_m<1>(mb);
+    case 2: return pick_mb_m<2>(mb);
     case 3: return pick_mb_m<3>(mb);
     case 4: return pick_mb_m<4>(mb);
     case 5: return pick_mb_m<5>(mb);

@@ -270,8 +270,10 @@ qx_fn pick_qx(int qn) {
 // launch (the pipelined batched form does not: M = 2 4096x4096 5.2 / 7.1) and
 // rows are short (M = 4 1024x2560 7.4 / 5.7, M = 2 4096x5120 10.3 / 7.7, M = 4
 // 4096x6144 13.3 / 9.8; but M = 2 4096x7168 9.8 / 11.2, M = 4 1024x5120 7.3 /
-// 8.8).
-bool q4_0_mx_takes(const GemvArgs &a, int64_t M) {
+// 8.8).  Only in the AUTO variant: MI355X_VARIANT_DIGITS promises the fixed-point
+// arithmetic of the dot-unit forms.
+bool q4_0_mx_takes(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) {
+    if (ctx->kernel_variant != MI355X_VARIANT_AUTO || !form_is_auto(ctx, a.type)) return false;
     if (M >= 5) return a.K <= 4096 || a.N >= (a.K <= 8192 ? 4096 : 16384);
     const bool pipelined = a.K % 2048 == 0 && (a.K <= 4096 || M == 2);
     return !pipelined && (a.K <= 4096 || (a.N >= 4096 && a.K <= (M == 2 ? 5120 : 6144)));

@@ -120,9 +120,9 @@ int q4_0_mb_capacity(const mi355x_ctx *ctx, const GemvArgs &a);
 // null for the context's own tile buffer (grown with hipMalloc on demand).
 int launch_gemv_q4_0_mb(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int M,
                         void *fixed_tiles);
-// The same rows on the matrix cores, without a buffer, and whether that form is
-// the faster one for a call of M activations.
-bool q4_0_mx_takes(const GemvArgs &a, int64_t M);
+// The same rows on the matrix cores, without a buffer, and whether a call of M
+// activations takes that form.
+bool q4_0_mx_takes(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M);
 int launch_gemv_q4_0_mx(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int M);
 // Device address of the static scratch on `device` (the device must be
 // current); resolved once per device with hipGetSymbolAddress.
@@ -154,6 +154,14 @@ bool kq_digit_rows(const mi355x_ctx *ctx, int type, int64_t N, int64_t K);
 // that is the fastest form for these sizes.
 bool kq_mx_takes(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M);
 int launch_gemv_kq_mx(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int M);
+
+// Whether the caller leaves the kernels' form to the library.  A form, rows per
+// step, wavefronts per workgroup (Q4_0) or prefetch that the caller has set
+// belongs to the digit and f32 kernels, so batched calls run those then.
+inline bool form_is_auto(const mi355x_ctx *ctx, int type) {
+    return ctx->form_override == MI355X_FORM_AUTO && ctx->rows_override == 0 && ctx->prefetch_override == 0 &&
+           (type != MI355X_TYPE_Q4_0 || ctx->waves_override == 0);
+}
 
 // Prepack kernels: byte-range scatter/gather between ggml and resident order.
 int launch_prepack_scatter(mi355x_ctx *ctx, int type, int64_t N, int64_t K, uint8_t *packed,

@@ -956,7 +956,7 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
         const int cap = q4_0_mb_capacity(ctx, a);
         if (cap >= 2) {
             DeviceGuard dg(ctx->device);
-            const bool mx = q4_0_mx_takes(a, M);
+            const bool mx = q4_0_mx_takes(ctx, a, M);
             for (int64_t m0 = 0; m0 < M;) {
                 const int chunk = static_cast<int>(std::min<int64_t>(cap, M - m0));
                 GemvArgs c{type, static_cast<const uint8_t *>(W), N, K, x + m0 * x_stride, false, y + m0 * y_stride};
