@@ -303,7 +303,11 @@ MI355X_API int mi355x_gemv_bf16(mi355x_ctx *ctx, int type, const void *W, int64_
  * context buffer, one batched launch; or one launch).  Other cases: M
  * sequential GEMVs; so are calls on a context whose form, rows, wavefronts
  * (Q4_0) or prefetch option is set, but for the digit-plane Q4_0 forms, and
- * calls of many activations with MI355X_OPT_GRID set.  Calls on one context
+ * calls of many activations with MI355X_OPT_GRID set.  While the context's
+ * stream records a HIP graph, many activations run without the workspace too
+ * (passes of 8 Q4_0 activations, M sequential GEMVs of the other types), so that
+ * a graph's replays on any stream share nothing with the context's other calls
+ * but the digit-plane Q4_0 form's activation buffer.  Calls on one context
  * serialise on its lock while they enqueue. */
 MI355X_API int mi355x_gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
                                    const float *x, int64_t x_stride, float *y, int64_t y_stride,
@@ -312,8 +316,9 @@ MI355X_API int mi355x_gemv_batched(mi355x_ctx *ctx, int type, const void *W, int
 /* Allocation-free form of mi355x_gemv_batched, for callers that cannot call
  * hipMalloc (code under HIP graph capture, tight serving loops, harnesses
  * that forbid it).  No counterpart in the reference.  Same arguments and the
- * same outputs, bit for bit; the matrix-core forms are the same launches (the
- * workspace is the context's from its creation); the K-split batched form
+ * same outputs, bit for bit (both under capture or both not); the matrix-core
+ * forms are the same launches (the workspace is the context's from its
+ * creation); the K-split batched form
  * keeps its activation tiles in the library's static device scratch of
  * MI355X_NOALLOC_SCRATCH_BYTES (336 KiB per device, held until the process
  * ends; enough for 8 activations of K = 16384 per pass, the most the form

@@ -911,10 +911,21 @@ bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) 
     return M >= (a.N < 4096 && !kq_digit_rows(ctx, a.type, a.N, a.K) ? 5 : 4);
 }
 
+// Whether the launches of a call now run in order on the context's stream, and
+// on no other: false while the stream records a graph.
+int gemm_batched_in_order(const mi355x_ctx *ctx, bool *in_order) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    MI355X_HIP(hipStreamIsCapturing(ctx->stream, &st));
+    *in_order = st == hipStreamCaptureStatusNone;
+    return MI355X_OK;
+}
+
 // The workspace belongs to the context from its creation to its end and never
-// moves, so no call allocates and a captured call stays valid; the context's
-// lock keeps the launches that share it together on its stream.  Activations
-// that it cannot hold at once go in several passes.
+// moves, so no call allocates; the context's lock keeps the launches that share
+// it together on its stream.  Activations that it cannot hold at once go in
+// several passes.  A graph may be replayed on any stream, at the same time as
+// the context's own calls, so a call under capture takes a form without the
+// workspace instead (gemm_batched_in_order).
 int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int64_t M_total) {
     const bool q40 = a.type == MI355X_TYPE_Q4_0;
     GemmArgs g{};

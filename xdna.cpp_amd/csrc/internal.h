@@ -129,9 +129,11 @@ int launch_gemv_q4_0_mx(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
 int resolve_scratch(int device, void **out);
 size_t scratch_bytes();
 // Matrix-core form of a batched call (any weight type): whether it takes M
-// activation rows of `a`, and its launches.
+// activation rows of `a`, whether its shared workspace is safe for the call (not
+// while the context's stream records a graph), and its launches.
 constexpr size_t kGemmWorkspace = size_t(64) << 20;
 bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M);
+int gemm_batched_in_order(const mi355x_ctx *ctx, bool *in_order);
 int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int64_t M);
 // Several Q4_0 matrices that share the activation row x as one launch of
 // the pipelined form (*launched = false where that form does not apply: the

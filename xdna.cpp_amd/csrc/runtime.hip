@@ -943,7 +943,12 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
         }
         GemvArgs a{type, static_cast<const uint8_t *>(W), N, K, x, false, y};
         if (kq_mx_takes(ctx, a, M)) return launch_gemv_kq_mx(ctx, a, x_stride, y_stride, static_cast<int>(M));
-        if (gemm_batched_supports(ctx, a, M)) return launch_gemm_batched(ctx, a, x_stride, y_stride, M);
+        if (gemm_batched_supports(ctx, a, M)) {
+            bool in_order = false;
+            rc = gemm_batched_in_order(ctx, &in_order);
+            if (rc) return rc;
+            if (in_order) return launch_gemm_batched(ctx, a, x_stride, y_stride, M);
+        }
     }
     // Q4_0: up to q4_0_mb_capacity() activations per launch (weights read once
     // per launch), on the matrix cores or in digit-plane arithmetic
