@@ -35,3 +35,30 @@ def check_gemv(y, y_ref, row_norms, x, what="") -> dict:
     assert c >= COS_MIN, f"{what}: cosine {c:.9f} < {COS_MIN} ({stats})"
     assert np.all(err <= bound), (f"{what}: row {worst} err {err[worst]:.3e} > bound {bound[worst]:.3e}")
     return stats
+
+
+# Results of f32-accurate arithmetic (f32 or 22-bit activations, f32 sums)
+# against 64 bits: per output at most F32_SUM * ||w|| * rms(x), the standard
+# deviation of an output whose activations are independent.  22-bit activations
+# are off by at most 2^-23 each (rms 4e-8 of that scale), a chain of f32 sums of
+# this length by 1e-7 to 2.5e-7; the bound is eight times that.  One f16 plane
+# alone (2^-12 at worst, rms 1e-4) exceeds it everywhere, 20-bit fixed point
+# per 32 values (rms 3e-6) and 16-bit (3e-5) on most outputs.
+F32_SUM = 2e-6
+
+
+def product64(oracle, t, raw, N, K, xs, grid=None):
+    """(xs @ W^T, ||w|| per row) in float64 from the oracle's weights."""
+    rows = np.ascontiguousarray(raw).reshape(N, -1)
+    W = np.stack([oracle.dequant_row(t, r, K, grid=grid) for r in rows]).astype(np.float64)
+    return np.asarray(xs, np.float64) @ W.T, np.linalg.norm(W, axis=1)
+
+
+def check_f32_sum(y, ref, norms, xs, what=""):
+    xs = np.asarray(xs, np.float64)
+    bound = F32_SUM * np.sqrt((xs * xs).mean(axis=1))[:, None] * norms[None, :]
+    err = np.abs(np.asarray(y, np.float64) - ref)
+    assert np.isfinite(err).all(), what
+    worst = float((err / np.maximum(bound, 1e-300)).max()) if err.size else 0.0
+    assert worst <= 1.0, f"{what}: {worst:.2f} times the bound"
+    return worst

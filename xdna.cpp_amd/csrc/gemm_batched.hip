@@ -17,7 +17,13 @@
 // of the row's largest value.  Products are exact in f32 and sums are f32 over
 // 256 values (32 for Q4_0), scaled by the superblock's d and added in f32 over
 // superblocks.  This is more accurate than the 20- or 16-bit fixed point of
-// the single-row kernels.
+// the single-row kernels, except that those scale every 32 values by themselves:
+// a row with a block of 32 whose largest value is more than 2^18 below the
+// row's is wide, and a wavefront sums wide rows in f32 after its tiles, four to
+// a pass over its weights, from the activations as they are.  (us with none, one
+// and all of the rows wide: Q4_0 17408x5120 M = 37 50, 85, 406; IQ3_S 8192x8192
+// M = 64 48, 75, 458.  Every row's activations go through the vector memory
+// path for 64 weight rows at a time, which bounds it.)
 //
 // Work split.  A workgroup of 4 wavefronts computes 256 output columns (weight
 // rows) x 32 or 64 activation rows; a wavefront 64 columns as two 32-wide
@@ -73,7 +79,9 @@ struct GemmArgs {
     int nseg;
     const uint8_t *planes;  // [superblock][half][Mp][512]
     const _Float16 *sums;   // [superblock][Mp][16]
-    const float *unit;      // [Mp]: 1 / s of each row
+    const float *unit;      // [Mp]: 1 / s of each row, negative for wide rows
+    const float *x;         // the activations themselves, for wide rows
+    int64_t x_stride;
     float *out;             // y, or the partials of segment 0
     int64_t out_stride;
     int64_t seg_stride;
@@ -183,7 +191,12 @@ __device__ __forceinline__ void store_superblock(const XPlanes &c, int m, int la
 
 // Planes, sums and units of the activation rows: one workgroup per row, its
 // wavefronts taking the superblocks in turn; the first kPlKeep of each stay in
-// registers between the row's maximum and the conversion.
+// registers between the row's maximum and the conversion.  A row is wide if a
+// block of 32 has a largest scaled value below kWideBelow but not 0: the planes
+// hold a value to 2^-25 at worst, which is then more than 2^-21 of the block's
+// largest (20-bit fixed point: 2^-20).
+constexpr float kWideBelow = 0.0625f;
+constexpr int kWideRows = 4;
 constexpr int kPlThreads = 1024, kPlWavesG = kPlThreads / 64, kPlKeep = 4;
 __global__ __launch_bounds__(kPlThreads) void gemm_planes_kernel(const float *x, int64_t x_stride, int64_t K,
                                                                  int x_al16, int Mp, int B, uint8_t *planes,
@@ -210,8 +223,13 @@ __global__ __launch_bounds__(kPlThreads) void gemm_planes_kernel(const float *x,
     mx = wave_max(smax[lane & (kPlWavesG - 1)]);
     float u;
     const float s = row_scale(mx, u);
-    if (threadIdx.x == 0) unit[m] = u;
+    int wide = 0;
     auto put = [&](int b, const float4 &f) {
+        float bm = abs_max4(f) * s;  // of the block, in its 8 lanes
+        bm = fmaxf(bm, dpp_mov<0xB1>(bm));
+        bm = fmaxf(bm, dpp_mov<0x4E>(bm));
+        bm = fmaxf(bm, dpp_mov<0x141>(bm));
+        wide |= bm > 0.f && bm < kWideBelow;
         uint8_t *h0 = planes + (static_cast<int64_t>(2 * b) * Mp + m) * kGmHalfBytes;
         store_superblock(convert_superblock(f, s), m, lane, h0, h0 + static_cast<int64_t>(Mp) * kGmHalfBytes,
                          sums + (static_cast<int64_t>(b) * Mp + m) * 16);
@@ -222,6 +240,8 @@ __global__ __launch_bounds__(kPlThreads) void gemm_planes_kernel(const float *x,
         if (b < B) put(b, keep[k]);
     }
     for (int b = wave + kPlWavesG * kPlKeep; b < B; b += kPlWavesG) put(b, load(b));
+    wide = __syncthreads_or(wide);
+    if (threadIdx.x == 0) unit[m] = wide ? -u : u;
 }
 
 // ---- weight decode --------------------------------------------------------------
@@ -281,6 +301,13 @@ __device__ __forceinline__ f16x8 k4_mins(const u32x4 &hd) {
     const f16x2 k = h2s(1024.f);
     return frag8(u2(h2((m0 & 0x00FF00FFu) | kH1024) - k), u2(h2(((m0 >> 8) & 0x00FF00FFu) | kH1024) - k),
                  u2(h2((m1 & 0x00FF00FFu) | kH1024) - k), u2(h2(((m1 >> 8) & 0x00FF00FFu) | kH1024) - k));
+}
+
+// the mins of sub-blocks 2c (low byte) and 2c + 1
+__device__ __forceinline__ uint32_t min_pair_k4(int c, const u32x4 &hd) {
+    const uint32_t sh = 16u * static_cast<uint32_t>(c & 1);
+    const uint32_t b2 = hd[2] >> sh, c2 = hd[3] >> sh;
+    return c < 2 ? (b2 & 0x3F3Fu) : (((c2 >> 4) & 0x0F0Fu) | ((b2 >> 2) & 0x3030u));
 }
 
 template <>
@@ -549,32 +576,33 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
 
     // the wavefront's rows of the matrix as one buffer (empty past N)
     const int64_t rows = a.N - n0 < 32 * NT ? (a.N - n0 > 0 ? a.N - n0 : 0) : 32 * NT;
-    LaneRow lr[NT];
-    {
+    auto view = [&](int c, LaneRow (&v)[NT]) {  // of the lanes of column c of the tiles
         const uint8_t *base = a.W + (rows > 0 ? n0 : 0) * a.row_bytes;
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint8_t *>(base), 0, static_cast<uint32_t>(rows * a.row_bytes), kBufferWord3);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const uint32_t rl = 32 * t + col;
-            lr[t].rsrc = rsrc;
-            lr[t].base = rl * static_cast<uint32_t>(a.row_bytes);
+            const uint32_t rl = 32 * t + c;
+            v[t].rsrc = rsrc;
+            v[t].base = rl * static_cast<uint32_t>(a.row_bytes);
             if constexpr (!Q40) {
                 constexpr KqLayout L = kq_layout(TYPE);
-                const bool flipped = kq_row_flipped(reinterpret_cast<uintptr_t>(base) + lr[t].base);
+                const bool flipped = kq_row_flipped(reinterpret_cast<uintptr_t>(base) + v[t].base);
                 if constexpr (L.grouped) {
-                    lr[t].P[0] = static_cast<uint32_t>(a.B);
-                    lr[t].P[1] = flipped ? 1u : 0u;
+                    v[t].P[0] = static_cast<uint32_t>(a.B);
+                    v[t].P[1] = flipped ? 1u : 0u;
                 } else {
 #pragma unroll
                     for (int i = 0; i < 5; ++i)
-                        lr[t].P[i] = i < L.nfields ? static_cast<uint32_t>(kq_plane_start(L, i, a.B, flipped)) : 0u;
+                        v[t].P[i] = i < L.nfields ? static_cast<uint32_t>(kq_plane_start(L, i, a.B, flipped)) : 0u;
                 }
             }
         }
-    }
+    };
+    LaneRow lr[NT];
+    view(col, lr);
     // raw weights of slice (or blocks) 4 half + 2q + h of superblock b
-    auto load_raw = [&](Regs (&r)[NT], int b, int half, int q) {
+    auto load_rows = [&](const LaneRow (&lr)[NT], int h, Regs (&r)[NT], int b, int half, int q) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             if constexpr (Q40) {
@@ -597,6 +625,8 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
             }
         }
     };
+
+    auto load_raw = [&](Regs (&r)[NT], int b, int half, int q) { load_rows(lr, h, r, b, half, q); };
 
     f32x16 acc[NT][MT];
     auto clear = [&] {
@@ -777,6 +807,7 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
                 const int m = m0 + 32 * i + 8 * (k >> 2) + 4 * h + (k & 3);
                 if (m >= a.M) continue;
                 const float u = a.unit[m];
+                if (u < 0.f) continue;  // a wide row
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     const int64_t n = n0 + 32 * t + col;
@@ -789,6 +820,142 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
 
     using H0 = std::integral_constant<int, 0>;
     using H1 = std::integral_constant<int, 1>;
+
+    // Wide activation rows m[0..] in f32, over superblocks [b0, b1), up to
+    // kWideRows in one pass over the weights: a lane sums its own slices of its
+    // weight rows from the operands that the products take.  (Everything of the
+    // lane is formed again here, from its number: nothing stays in registers for
+    // this over the products.)
+    auto wide_rows = [&](int lane, const int (&m)[kWideRows], int b0, int b1, float *out) {
+        const int col = lane & 31, h = lane >> 5;
+        LaneRow lr[NT];
+        view(col, lr);
+        const float *x[kWideRows];
+#pragma unroll
+        for (int r = 0; r < kWideRows; ++r) x[r] = a.x + m[r] * a.x_stride;
+        float wacc[kWideRows][NT] = {};
+        // an operand's dwords as its 8 values in order
+        auto widen = [](const uint32_t (&w)[4], float (&f)[8]) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                f[4 * (j >> 1) + (j & 1)] = static_cast<float>(h2(w[j])[0]);
+                f[4 * (j >> 1) + (j & 1) + 2] = static_cast<float>(h2(w[j])[1]);
+            }
+        };
+        auto dot8 = [](const float (&w)[8], const float (&v)[8]) {
+            return (fmaf(w[0], v[0], w[1] * v[1]) + fmaf(w[2], v[2], w[3] * v[3])) +
+                   (fmaf(w[4], v[4], w[5] * v[5]) + fmaf(w[6], v[6], w[7] * v[7]));
+        };
+        auto load8 = [&](int r, int64_t i, float (&v)[8]) {
+            __builtin_memcpy(&v[0], x[r] + i, 16);
+            __builtin_memcpy(&v[4], x[r] + i + 4, 16);
+        };
+        for (int b = b0; b < b1; ++b) {
+            float sup[kWideRows][NT] = {}, low[kWideRows][NT] = {}, d[NT], dm[NT];
+            auto quarter = [&](auto HALF, auto Q) {
+                constexpr int half = decltype(HALF)::value, q = decltype(Q)::value;
+                Regs g[NT];
+                load_rows(lr, h, g, b, half, q);
+                float v[8];
+                if constexpr (Q40) {
+                    const int blk = 8 * b + 4 * half + 2 * q;
+                    if (blk >= a.blocks) return;
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        float s[kWideRows][NT] = {};
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            float f[NT][8];
+#pragma unroll
+                            for (int t = 0; t < NT; ++t) {
+                                uint32_t w[4];
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) w[j] = q40_dword(g[t], e, i, j);
+                                widen(w, f[t]);
+                            }
+#pragma unroll
+                            for (int r = 0; r < kWideRows; ++r) {
+                                load8(r, 32 * static_cast<int64_t>(blk + e) + 16 * i + 8 * h, v);
+#pragma unroll
+                                for (int t = 0; t < NT; ++t) s[r][t] += dot8(f[t], v);
+                            }
+                        }
+#pragma unroll
+                        for (int r = 0; r < kWideRows; ++r)
+#pragma unroll
+                            for (int t = 0; t < NT; ++t) sup[r][t] = fmaf(half_f(g[t].d[e]), s[r][t], sup[r][t]);
+                    }
+                } else {
+                    constexpr int SH = slice_shape(TYPE);
+                    constexpr bool MINS = Gw<TYPE>::kMins;
+                    float sx[MINS ? kWideRows : 1][2] = {};  // of positions 0, 1 and 2, 3
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {
+                        float f[NT][8], rest[NT][8];
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) {
+                            uint2 e[2] = {};
+#pragma unroll
+                            for (int k = 0; k < Gw<TYPE>::kLooks; ++k) {
+                                if constexpr (Gw<TYPE>::kLooks > 0) e[k] = Gw<TYPE>::look(g[t], p, k, tab);
+                            }
+                            uint32_t w[4], l[4] = {};
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) Gw<TYPE>::dword(g[t], half, q, p, j, e, w[j], l[j]);
+                            widen(w, f[t]);
+                            if constexpr (Gw<TYPE>::kWide) {
+                                widen(l, rest[t]);
+#pragma unroll
+                                for (int i = 0; i < 8; ++i) f[t][i] += rest[t][i];  // exact: 12 bits
+                            }
+                        }
+#pragma unroll
+                        for (int r = 0; r < kWideRows; ++r) {
+                            load8(r, 256 * static_cast<int64_t>(b) + 128 * half + 8 * run_of<SH>(2 * q + h, p), v);
+                            if constexpr (MINS)
+                                sx[r][p >> 1] += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+#pragma unroll
+                            for (int t = 0; t < NT; ++t) sup[r][t] += dot8(f[t], v);
+                        }
+                    }
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        d[t] = Gw<TYPE>::d(g[t]);
+                        if constexpr (MINS) {
+                            const uint32_t mn = min_pair_k4(2 * half + q, g[t].hd);
+                            const float m0 = static_cast<float>(mn & 0xFFu), m1 = static_cast<float>(mn >> 8);
+#pragma unroll
+                            for (int r = 0; r < kWideRows; ++r) low[r][t] += fmaf(m0, sx[r][0], m1 * sx[r][1]);
+                            dm[t] = half_f(g[t].hd[0] >> 16);
+                        }
+                    }
+                }
+            };
+            quarter(H0{}, H0{});
+            __builtin_amdgcn_sched_barrier(0);
+            quarter(H0{}, H1{});
+            __builtin_amdgcn_sched_barrier(0);
+            quarter(H1{}, H0{});
+            __builtin_amdgcn_sched_barrier(0);
+            quarter(H1{}, H1{});
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < kWideRows; ++r)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    if constexpr (Q40) wacc[r][t] += sup[r][t];
+                    else if constexpr (Gw<TYPE>::kMins) wacc[r][t] += fmaf(d[t], sup[r][t], -dm[t] * low[r][t]);
+                    else wacc[r][t] = fmaf(d[t], sup[r][t], wacc[r][t]);
+                }
+        }
+        static_assert(NT == 2, "lane half h stores column tile h");
+        const int64_t n = n0 + 32 * h + col;
+#pragma unroll
+        for (int r = 0; r < kWideRows; ++r) {
+            const float y0 = wacc[r][0] + __shfl_xor(wacc[r][0], 32), y1 = wacc[r][1] + __shfl_xor(wacc[r][1], 32);
+            if (n < a.N) out[m[r] * a.out_stride + n] = h ? y1 : y0;
+        }
+    };
     stage_table<TYPE>(a, tab);
     vlast = f32x16{};
 
@@ -833,6 +1000,20 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     }
     flush();
     store(seg);
+    uint32_t ones = ~0u;
+    asm volatile("" : "+s"(ones));
+    const int lid = static_cast<int>(__builtin_amdgcn_mbcnt_hi(ones, __builtin_amdgcn_mbcnt_lo(ones, 0u)));
+    const int ml = m0 + (lid & (BM - 1));
+    uint64_t wide = __ballot(lid < BM && ml < a.M && a.unit[ml] < 0.f);
+    while (wide) {
+        int m[kWideRows];  // the last one repeats
+#pragma unroll
+        for (int r = 0; r < kWideRows; ++r) {
+            m[r] = wide ? m0 + __builtin_ctzll(wide) : m[r > 0 ? r - 1 : 0];
+            wide &= wide - 1;
+        }
+        wide_rows(lid, m, b0, b1, a.out + seg * a.seg_stride);
+    }
 }
 
 // y = partial 0 + partial 1 + ..., in segment order
@@ -962,13 +1143,15 @@ int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
         uint8_t *p = static_cast<uint8_t *>(ctx->gemm_buf);
         g.planes = p;
         g.sums = reinterpret_cast<const _Float16 *>(p + planes_bytes(g.B, g.Mp));
+        g.x = static_cast<const float *>(a.x) + mb * x_stride;
+        g.x_stride = x_stride;
         g.unit = reinterpret_cast<const float *>(p + planes_bytes(g.B, g.Mp) + sums_bytes(g.B, g.Mp));
         float *partial = reinterpret_cast<float *>(p + staged);
         g.out = g.nseg > 1 ? partial : y;
         g.out_stride = g.nseg > 1 ? a.N : y_stride;
         g.seg_stride = static_cast<int64_t>(M) * a.N;
         hipLaunchKernelGGL(gemm_planes_kernel, dim3(static_cast<unsigned>(M)), dim3(kPlThreads), 0, ctx->stream,
-                           static_cast<const float *>(a.x) + mb * x_stride, x_stride, a.K, x_al16, g.Mp, g.B, p,
+                           g.x, x_stride, a.K, x_al16, g.Mp, g.B, p,
                            const_cast<_Float16 *>(g.sums), const_cast<float *>(g.unit));
         MI355X_HIP(hipGetLastError());
         hipLaunchKernelGGL(pick_gemm(a.type, mt), dim3(grid_x, static_cast<unsigned>(g.nseg)), dim3(kGmThreads), 0,
