@@ -10,20 +10,21 @@
 // Arithmetic.  Codes times integer sub-block scales are exact in f16 (11
 // bits) for Q3_K, Q4_K, Q5_K, IQ3_S, and for IQ3_XXS / IQ2_S with grids up to
 // 66; Q6_K and IQ4_XS need 12 bits and take a second operand with the exact
-// remainder; Q4_0 keeps its bare codes and applies the block scale to each
-// block's sum.  Activations are split into two f16 planes, hi = f16(x s) and
-// lo = f16(x s - hi) with s a power of two per row that puts its largest |x|
-// in [2^14, 2^15): x s = hi + lo to 2^-22 of x, or 2^-25 absolute, i.e. 2^-39
-// of the row's largest value.  Products are exact in f32 and sums are f32 over
-// 256 values (32 for Q4_0), scaled by the superblock's d and added in f32 over
-// superblocks.  This is more accurate than the 20- or 16-bit fixed point of
-// the single-row kernels, except that those scale every 32 values by themselves:
-// a row with a block of 32 whose largest value is more than 2^18 below the
-// row's is wide, and a wavefront sums wide rows in f32 after its tiles, four to
-// a pass over its weights, from the activations as they are.  (us with none, one
-// and all of the rows wide: Q4_0 17408x5120 M = 37 50, 85, 406; IQ3_S 8192x8192
-// M = 64 48, 75, 458.  Every row's activations go through the vector memory
-// path for 64 weight rows at a time, which bounds it.)
+// remainder, which meets the activations' high plane only (its product with the
+// low one is at most 2^-22 of the term); Q4_0 keeps its bare codes and applies
+// the block scale to each block's sum.  Activations are split into two f16
+// planes, hi = f16(x s) and lo = f16(x s - hi) with s a power of two per row that
+// puts its largest |x| in [2^14, 2^15): x s = hi + lo to 2^-23 of x, or 2^-25
+// absolute, i.e. 2^-39 of the row's largest value.  Products are exact in f32 and
+// sums are f32 over 256 values (32 for Q4_0), scaled by the superblock's d and
+// added in f32 over superblocks (FINE kernels: in f64).  This is more accurate
+// than the 20- or 16-bit fixed point of the single-row kernels, except that those
+// scale every 32 values by themselves: a row with a block of 32 whose largest
+// value is more than 2^18 below the row's is wide, and a wavefront sums wide rows
+// in f32 after its tiles, four to a pass over its weights, from the activations
+// as they are.  (us with none, one and all of the rows wide: Q4_0 17408x5120 M =
+// 37 50, 85, 406; IQ3_S 8192x8192 M = 64 48, 75, 458.  Every row's activations go
+// through the vector memory path for 64 weight rows at a time, which bounds it.)
 //
 // Work split.  A workgroup of 4 wavefronts computes 256 output columns (weight
 // rows) x 32 or 64 activation rows; a wavefront 64 columns as two 32-wide
@@ -194,13 +195,13 @@ __device__ __forceinline__ void store_superblock(const XPlanes &c, int m, int la
 // registers between the row's maximum and the conversion.  A row is wide if a
 // block of 32 has a largest scaled value below kWideBelow but not 0: the planes
 // hold a value to 2^-25 at worst, which is then more than 2^-21 of the block's
-// largest (20-bit fixed point: 2^-20).
-constexpr float kWideBelow = 0.0625f;
+// largest (20-bit fixed point: 2^-20), or than 2^-25 where f32 is the measure.
+constexpr float kWideBelow = 0.0625f, kWideBelowF32 = 1.0f;
 constexpr int kWideRows = 4;
 constexpr int kPlThreads = 1024, kPlWavesG = kPlThreads / 64, kPlKeep = 4;
 __global__ __launch_bounds__(kPlThreads) void gemm_planes_kernel(const float *x, int64_t x_stride, int64_t K,
-                                                                 int x_al16, int Mp, int B, uint8_t *planes,
-                                                                 _Float16 *sums, float *unit) {
+                                                                 int x_al16, float wide_below, int Mp, int B,
+                                                                 uint8_t *planes, _Float16 *sums, float *unit) {
     __shared__ float smax[kPlWavesG];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, m = blockIdx.x;
     const float *xr = x + m * x_stride;
@@ -229,7 +230,7 @@ __global__ __launch_bounds__(kPlThreads) void gemm_planes_kernel(const float *x,
         bm = fmaxf(bm, dpp_mov<0xB1>(bm));
         bm = fmaxf(bm, dpp_mov<0x4E>(bm));
         bm = fmaxf(bm, dpp_mov<0x141>(bm));
-        wide |= bm > 0.f && bm < kWideBelow;
+        wide |= bm > 0.f && bm < wide_below;
         uint8_t *h0 = planes + (static_cast<int64_t>(2 * b) * Mp + m) * kGmHalfBytes;
         store_superblock(convert_superblock(f, s), m, lane, h0, h0 + static_cast<int64_t>(Mp) * kGmHalfBytes,
                          sums + (static_cast<int64_t>(b) * Mp + m) * 16);
@@ -554,10 +555,20 @@ __device__ __forceinline__ void gm_barrier() {
     __syncthreads();
 }
 
-template <int TYPE, int MT>
+// FINE: for calls whose one-row kernels sum f32 activations in f32 (IQ types).
+// The low planes' products have sums of their own, so that they do not add
+// roundings at the size of the high ones', and the sums of each half superblock
+// (IQ2_S: quarter) are added in f64.  Error against 64 bits over K = 256 to 16384
+// and N = 64 to 12000, f32 rows in brackets: IQ3_S and IQ3_XXS 1.0e-7 (1.2 to
+// 1.4e-7), IQ2_S 0.8 to 0.9e-7 (0.9 to 1.2e-7), IQ4_XS 1.05e-7 (2.5e-7); without
+// them 1.6 to 1.9e-7.  us, without -> with: IQ3_S 1024x4096 M = 9 18.9 -> 20.1,
+// M = 512 61 -> 75; IQ2_S 17408x11008 M = 128 164 -> 331 (one GEMV each: 37, 1993
+// and 4134).
+template <int TYPE, int MT, bool FINE>
 __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     constexpr int BM = 32 * MT, NT = kGmNT;
     constexpr bool Q40 = TYPE == MI355X_TYPE_Q4_0;
+    constexpr bool MINS = TYPE == MI355X_TYPE_Q4_K || TYPE == MI355X_TYPE_Q5_K;
     using Regs = typename RegsOf<TYPE>::T;
     __shared__ uint4 xh0[BM * kGmHalfBytes / 16], xh1[BM * kGmHalfBytes / 16];
     __shared__ uint4 ssum[2][BM * 2];
@@ -629,11 +640,18 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     auto load_raw = [&](Regs (&r)[NT], int b, int half, int q) { load_rows(lr, h, r, b, half, q); };
 
     f32x16 acc[NT][MT];
+    double accd[FINE ? NT : 1][FINE ? MT : 1][16];
     auto clear = [&] {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int i = 0; i < MT; ++i) acc[t][i] = f32x16{};
+            for (int i = 0; i < MT; ++i) {
+                acc[t][i] = f32x16{};
+                if constexpr (FINE) {
+#pragma unroll
+                    for (int k = 0; k < 16; ++k) accd[t][i][k] = 0.0;
+                }
+            }
     };
     const int mx = col & 15;  // the rows' slot swizzle (m0 is a multiple of 32)
     auto operand = [&](const uint4 *xb, int plane, int run, int tile) {
@@ -654,6 +672,7 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     u32x4 bw[Q40 ? NT : 1][2][2];                    // Q4_0: the block's two operands
     float bd[NT][2];
     f32x16 tsum[Q40 ? 1 : NT][Q40 ? 1 : MT];
+    f32x16 tlow[FINE ? NT : 1][FINE ? MT : 1];
     f32x16 vlast;
     float dlast = 0.f;
     auto op = [](const u32x4 &v) { return __builtin_bit_cast(f16x8, v); };
@@ -696,6 +715,22 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
         }
     };
 
+    // FINE: the sums of a half superblock (IQ2_S: of each quarter, as its f32 rows
+    // are the most accurate)
+    constexpr bool QUARTERS = FINE && TYPE == MI355X_TYPE_IQ2_S;
+    auto finish_fine = [&](const Regs (&r)[NT]) {
+        if constexpr (FINE) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const double d = static_cast<double>(Gw<TYPE>::d(r[t]));
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int k = 0; k < 16; ++k)
+                        accd[t][i][k] = fma(d, static_cast<double>(tsum[t][i][k] + tlow[t][i][k]), accd[t][i][k]);
+            }
+        }
+    };
     // One half superblock from its raw weights r, its first operands already
     // decoded; `refill` loads r[0] of the next half once this one's are
     // decoded, and the last step decodes that half's first operands.
@@ -743,14 +778,17 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
             for (int k = 0; k < 2 * MT; ++k) x[0][k] = read(0, k);
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
+                if (QUARTERS && s == 4) finish_fine(r[0]);
                 if (s == 4) refill();  // r[0] is decoded; after the wait for r[1]'s loads in step 3
                 const int n = (s + 1) & 7, nh = s < 7 ? half : 1 - half;
 #pragma unroll
                 for (int m = 0; m < NM; ++m) {
                     const int plane = m / TM, i = m / NT % MT, t = m % NT;
-                    const bool first = half == 0 && s == 0 && plane == 0;
-                    tsum[t][i] = mfma(x[s & 1][2 * i + (plane == 1)], op(plane == 2 ? fl[t][s & 1] : fw[t][s & 1]),
-                                      first ? f32x16{} : tsum[t][i]);
+                    const bool low = FINE && plane > 0;
+                    const bool first = (half == 0 || FINE) && (s == 0 || (QUARTERS && s == 4)) && (low ? plane == 1 : plane == 0);
+                    f32x16 &c = low ? tlow[FINE ? t : 0][FINE ? i : 0] : tsum[t][i];
+                    c = mfma(x[s & 1][2 * i + (plane == 1)], op(plane == 2 ? fl[t][s & 1] : fw[t][s & 1]),
+                             first ? f32x16{} : c);
                     if (s < 7 && m < 2 * MT) x[(s + 1) & 1][m] = read(s + 1, m);
                     // the next step's operands, 4 NT dwords over NM products,
                     // and the table entries of the one after
@@ -767,7 +805,7 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     };
     // K types, end of a superblock: acc += d * tsum - dmin * mins . sums
     auto finish = [&](const Regs (&r)[NT], int par) {
-        if constexpr (!Q40) {
+        if constexpr (!Q40 && !FINE) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 const float d = Gw<TYPE>::d(r[t]);
@@ -812,7 +850,8 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
                 for (int t = 0; t < NT; ++t) {
                     const int64_t n = n0 + 32 * t + col;
                     if (n >= a.N) continue;
-                    out[m * a.out_stride + n] = u * acc[t][i][k];
+                    if constexpr (FINE) out[m * a.out_stride + n] = static_cast<float>(static_cast<double>(u) * accd[t][i][k]);
+                    else out[m * a.out_stride + n] = u * acc[t][i][k];
                 }
             }
         }
@@ -833,7 +872,7 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
         const float *x[kWideRows];
 #pragma unroll
         for (int r = 0; r < kWideRows; ++r) x[r] = a.x + m[r] * a.x_stride;
-        float wacc[kWideRows][NT] = {};
+        double wacc[kWideRows][NT] = {};
         // an operand's dwords as its 8 values in order
         auto widen = [](const uint32_t (&w)[4], float (&f)[8]) {
 #pragma unroll
@@ -887,7 +926,6 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
                     }
                 } else {
                     constexpr int SH = slice_shape(TYPE);
-                    constexpr bool MINS = Gw<TYPE>::kMins;
                     float sx[MINS ? kWideRows : 1][2] = {};  // of positions 0, 1 and 2, 3
 #pragma unroll
                     for (int p = 0; p < 4; ++p) {
@@ -943,17 +981,18 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
             for (int r = 0; r < kWideRows; ++r)
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
-                    if constexpr (Q40) wacc[r][t] += sup[r][t];
-                    else if constexpr (Gw<TYPE>::kMins) wacc[r][t] += fmaf(d[t], sup[r][t], -dm[t] * low[r][t]);
-                    else wacc[r][t] = fmaf(d[t], sup[r][t], wacc[r][t]);
+                    float v = sup[r][t];
+                    if constexpr (!Q40) v *= d[t];
+                    if constexpr (MINS) v = fmaf(-dm[t], low[r][t], v);
+                    wacc[r][t] += static_cast<double>(v);
                 }
         }
         static_assert(NT == 2, "lane half h stores column tile h");
         const int64_t n = n0 + 32 * h + col;
 #pragma unroll
         for (int r = 0; r < kWideRows; ++r) {
-            const float y0 = wacc[r][0] + __shfl_xor(wacc[r][0], 32), y1 = wacc[r][1] + __shfl_xor(wacc[r][1], 32);
-            if (n < a.N) out[m[r] * a.out_stride + n] = h ? y1 : y0;
+            const double y0 = wacc[r][0] + __shfl_xor(wacc[r][0], 32), y1 = wacc[r][1] + __shfl_xor(wacc[r][1], 32);
+            if (n < a.N) out[m[r] * a.out_stride + n] = static_cast<float>(h ? y1 : y0);
         }
     };
     stage_table<TYPE>(a, tab);
@@ -964,7 +1003,6 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     auto half_src = [&](int b, int half) {
         return a.planes + (static_cast<int64_t>(2 * b + half) * a.Mp + m0) * kGmHalfBytes;
     };
-    constexpr bool MINS = TYPE == MI355X_TYPE_Q4_K || TYPE == MI355X_TYPE_Q5_K;
     // sums of superblock b (types with mins): threads 0 .. 2 BM - 1
     auto load_sums = [&](int b, uint4 &s) {
         if (MINS && threadIdx.x < 2 * BM)
@@ -988,12 +1026,14 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
         load_raw(r[1], b, 0, 1);
         __builtin_amdgcn_sched_barrier(0);  // the loads go out before this half's work
         half_step(r, xh0, H0{}, [&] { load_raw(r[0], b, 1, 0); });
+        finish_fine(r[1]);
         gm_barrier();
         copy_planes<BM>(half_src(bn, 0), xh0, wave, lane);
         load_sums(bn, s);
         load_raw(r[1], b, 1, 1);
         __builtin_amdgcn_sched_barrier(0);
         half_step(r, xh1, H1{}, [&] { load_raw(r[0], bn, 0, 0); });
+        finish_fine(r[1]);
         finish(r[1], b & 1);
         put_sums((b + 1) & 1, s);
         gm_barrier();
@@ -1016,16 +1056,16 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     }
 }
 
-// y = partial 0 + partial 1 + ..., in segment order
+// y = partial 0 + partial 1 + ..., in segment order, rounded once
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float *part, int64_t seg_stride, int nseg, int M,
                                                           int64_t N, float *y, int64_t y_stride) {
     const int64_t n = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (n >= N) return;
     for (int m = blockIdx.y; m < M; m += gridDim.y) {
         const float *p = part + m * N + n;
-        float v = p[0];
-        for (int s = 1; s < nseg; ++s) v += p[s * seg_stride];
-        y[m * y_stride + n] = v;
+        double v = p[0];
+        for (int s = 1; s < nseg; ++s) v += static_cast<double>(p[s * seg_stride]);
+        y[m * y_stride + n] = static_cast<float>(v);
     }
 }
 
@@ -1033,20 +1073,25 @@ typedef void (*gemm_fn)(GemmArgs);
 
 template <int TYPE>
 gemm_fn pick_gemm_type(int mt) {
-    return mt == 1 ? gemm_kernel<TYPE, 1> : gemm_kernel<TYPE, 2>;
+    return mt == 1 ? gemm_kernel<TYPE, 1, false> : gemm_kernel<TYPE, 2, false>;
+}
+// FINE tiles are of 32 activations: the second sums of 64 do not fit the registers
+template <int TYPE>
+gemm_fn pick_gemm_iq(int mt, bool fine) {
+    return fine ? gemm_kernel<TYPE, 1, true> : pick_gemm_type<TYPE>(mt);
 }
 
-gemm_fn pick_gemm(int type, int mt) {
+gemm_fn pick_gemm(int type, int mt, bool fine) {
     switch (type) {
     case MI355X_TYPE_Q4_0: return pick_gemm_type<MI355X_TYPE_Q4_0>(mt);
     case MI355X_TYPE_Q3_K: return pick_gemm_type<MI355X_TYPE_Q3_K>(mt);
     case MI355X_TYPE_Q4_K: return pick_gemm_type<MI355X_TYPE_Q4_K>(mt);
     case MI355X_TYPE_Q5_K: return pick_gemm_type<MI355X_TYPE_Q5_K>(mt);
     case MI355X_TYPE_Q6_K: return pick_gemm_type<MI355X_TYPE_Q6_K>(mt);
-    case MI355X_TYPE_IQ4_XS: return pick_gemm_type<MI355X_TYPE_IQ4_XS>(mt);
-    case MI355X_TYPE_IQ3_S: return pick_gemm_type<MI355X_TYPE_IQ3_S>(mt);
-    case MI355X_TYPE_IQ3_XXS: return pick_gemm_type<MI355X_TYPE_IQ3_XXS>(mt);
-    case MI355X_TYPE_IQ2_S: return pick_gemm_type<MI355X_TYPE_IQ2_S>(mt);
+    case MI355X_TYPE_IQ4_XS: return pick_gemm_iq<MI355X_TYPE_IQ4_XS>(mt, fine);
+    case MI355X_TYPE_IQ3_S: return pick_gemm_iq<MI355X_TYPE_IQ3_S>(mt, fine);
+    case MI355X_TYPE_IQ3_XXS: return pick_gemm_iq<MI355X_TYPE_IQ3_XXS>(mt, fine);
+    case MI355X_TYPE_IQ2_S: return pick_gemm_iq<MI355X_TYPE_IQ2_S>(mt, fine);
     default: return nullptr;
     }
 }
@@ -1055,7 +1100,7 @@ size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
 // Rows of activation tiles for M activations, and what their planes, sums and
 // units take of the workspace.
-int tile_rows(int M) { return M <= 32 ? 32 : (M + 63) / 64 * 64; }
+int tile_rows(int M, bool fine) { return M <= 32 || fine ? (M + 31) / 32 * 32 : (M + 63) / 64 * 64; }
 size_t planes_bytes(int64_t B, int Mp) { return static_cast<size_t>(B) * 2 * Mp * kGmHalfBytes; }
 size_t sums_bytes(int64_t B, int Mp) { return align256(static_cast<size_t>(B) * Mp * 32); }
 size_t staged_bytes(int64_t B, int Mp) {
@@ -1076,6 +1121,10 @@ size_t staged_bytes(int64_t B, int Mp) {
 bool gemm_batched_supports(const mi355x_ctx *ctx, const GemvArgs &a, int64_t M) {
     if (ctx->kernel_variant != MI355X_VARIANT_AUTO || !form_is_auto(ctx, a.type) || ctx->grid_override != 0) return false;
     if (a.x_bf16 || a.N <= 0 || a.K <= 0 || !ctx->gemm_buf) return false;
+    // Q4_0 rows past 16384 values have f32 one-row kernels (error against 64 bits
+    // 2.7e-7; here 1.7e-7 at 17408x16640 and 2.3e-7 at 17408x32768, growing with
+    // the f32 chain of a row's blocks)
+    if (a.type == MI355X_TYPE_Q4_0 && a.K > 32768) return false;
     // 32-bit offsets into the 64 rows of a wavefront
     const int64_t row_bytes = a.type == MI355X_TYPE_Q4_0 ? a.K / 32 * 18 : a.K / 256 * kq_layout(a.type).block_bytes;
     if (row_bytes <= 0 || row_bytes >= (int64_t(1) << 31) / 64 || a.N >= (int64_t(1) << 31)) return false;
@@ -1109,6 +1158,9 @@ int gemm_batched_in_order(const mi355x_ctx *ctx, bool *in_order) {
 // workspace instead (gemm_batched_in_order).
 int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, int64_t y_stride, int64_t M_total) {
     const bool q40 = a.type == MI355X_TYPE_Q4_0;
+    // calls that replace f32 rows
+    const bool f32_rows = q40 ? a.K > 16384 : !kq_digit_rows(ctx, a.type, a.N, a.K);
+    const bool fine = f32_rows && !q40;
     GemmArgs g{};
     g.W = a.W;
     g.N = a.N;
@@ -1124,10 +1176,10 @@ int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
     std::lock_guard<std::mutex> lk(ctx->mu);
     for (int64_t mb = 0; mb < M_total; mb += g.M) {
         int M = static_cast<int>(std::min<int64_t>(kGmMaxRows, M_total - mb));
-        while (M > 32 && staged_bytes(g.B, tile_rows(M)) > kGemmWorkspace) M = std::max(32, (M / 2 + 31) / 32 * 32);
-        const int mt = M <= 32 ? 1 : 2;
+        while (M > 32 && staged_bytes(g.B, tile_rows(M, fine)) > kGemmWorkspace) M = std::max(32, (M / 2 + 31) / 32 * 32);
+        const int mt = M <= 32 || fine ? 1 : 2;
         g.M = M;
-        g.Mp = tile_rows(M);
+        g.Mp = tile_rows(M, fine);
         g.mtiles = g.Mp / (32 * mt);
         float *y = a.y + mb * y_stride;
         const int64_t tiles = static_cast<int64_t>(g.ntiles) * g.mtiles;
@@ -1151,10 +1203,10 @@ int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
         g.out_stride = g.nseg > 1 ? a.N : y_stride;
         g.seg_stride = static_cast<int64_t>(M) * a.N;
         hipLaunchKernelGGL(gemm_planes_kernel, dim3(static_cast<unsigned>(M)), dim3(kPlThreads), 0, ctx->stream,
-                           g.x, x_stride, a.K, x_al16, g.Mp, g.B, p,
+                           g.x, x_stride, a.K, x_al16, f32_rows ? kWideBelowF32 : kWideBelow, g.Mp, g.B, p,
                            const_cast<_Float16 *>(g.sums), const_cast<float *>(g.unit));
         MI355X_HIP(hipGetLastError());
-        hipLaunchKernelGGL(pick_gemm(a.type, mt), dim3(grid_x, static_cast<unsigned>(g.nseg)), dim3(kGmThreads), 0,
+        hipLaunchKernelGGL(pick_gemm(a.type, mt, fine), dim3(grid_x, static_cast<unsigned>(g.nseg)), dim3(kGmThreads), 0,
                            ctx->stream, g);
         MI355X_HIP(hipGetLastError());
         if (g.nseg > 1) {
