@@ -840,12 +840,14 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
         float *out = a.out + seg * a.seg_stride;
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
+            float us[16];  // requested together, negative for wide rows
+#pragma unroll
+            for (int k = 0; k < 16; ++k) us[k] = a.unit[min(m0 + 32 * i + 8 * (k >> 2) + 4 * h + (k & 3), a.M - 1)];
 #pragma unroll
             for (int k = 0; k < 16; ++k) {
                 const int m = m0 + 32 * i + 8 * (k >> 2) + 4 * h + (k & 3);
-                if (m >= a.M) continue;
-                const float u = a.unit[m];
-                if (u < 0.f) continue;  // a wide row
+                const float u = us[k];
+                if (m >= a.M || u < 0.f) continue;
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     const int64_t n = n0 + 32 * t + col;
@@ -1056,15 +1058,17 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     }
 }
 
-// y = partial 0 + partial 1 + ..., in segment order, rounded once
+// y = partial 0 + partial 1 + ..., in segment order, in Sum (f64 for the FINE
+// kernels' partials, which costs 1.8 us more at 4 x 512 x 4096)
+template <class Sum>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float *part, int64_t seg_stride, int nseg, int M,
                                                           int64_t N, float *y, int64_t y_stride) {
     const int64_t n = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (n >= N) return;
     for (int m = blockIdx.y; m < M; m += gridDim.y) {
         const float *p = part + m * N + n;
-        double v = p[0];
-        for (int s = 1; s < nseg; ++s) v += static_cast<double>(p[s * seg_stride]);
+        Sum v = p[0];
+        for (int s = 1; s < nseg; ++s) v += static_cast<Sum>(p[s * seg_stride]);
         y[m * y_stride + n] = static_cast<float>(v);
     }
 }
@@ -1210,7 +1214,8 @@ int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
                            ctx->stream, g);
         MI355X_HIP(hipGetLastError());
         if (g.nseg > 1) {
-            hipLaunchKernelGGL(gemm_reduce_kernel, dim3(static_cast<unsigned>((a.N + 255) / 256), std::min(M, 64)),
+            hipLaunchKernelGGL(fine ? gemm_reduce_kernel<double> : gemm_reduce_kernel<float>,
+                               dim3(static_cast<unsigned>((a.N + 255) / 256), std::min(M, 64)),
                                dim3(256), 0, ctx->stream, partial, g.seg_stride, g.nseg, M, a.N, y, y_stride);
             MI355X_HIP(hipGetLastError());
         }
