@@ -51,3 +51,26 @@ def test_wide_rows(ctx, oracle, name, N, K, M):
     # the other rows do not notice
     plain = [m for m in range(M) if m not in (1, 4, M - 1)]
     assert np.array_equal(run(ctx, t, raw, N, K, base)[plain], y[plain])
+
+
+# few Q4_0 activations: one quad of blocks and several per wavefront, wavefronts
+# without a quad, two launches (K > 8192), more tiles than workgroups, passes of 8
+@pytest.mark.parametrize("N,K,M", [(50, 256, 2), (300, 1024, 5), (17, 2560, 3), (4100, 8192, 8), (16400, 9216, 5),
+                                   (16 * 600 + 5, 1024, 8), (70, 2048, 13)])
+def test_few_wide_q4_0_rows(ctx, oracle, N, K, M):
+    raw = zero_scales(2, synth.random_q4_0(N, K, N + K), N, [0, K // 32 - 1])
+    base = np.stack([synth.activations(K, seed=50 + m) for m in range(M)])
+    base[:, :32] = base[:, -32:] = 0
+    base[0, 64:128] = 0  # blocks of zeros are not small
+    xs = base.copy()
+    xs[1, 3] = 2.0 ** 24
+    xs[M - 1] *= 2.0 ** -60
+    xs[M - 1, K - 1] = 2.0 ** 60
+    scale = np.ones((M, 1))
+    scale[M - 1] = 2.0 ** -60
+    rows = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(0, N - 40), N)]))
+    ref, norms = product64(oracle, 2, raw[rows], len(rows), K, base)
+    y = run(ctx, 2, raw, N, K, xs)
+    check_f32_sum(y[:, rows] / scale, ref, norms, base, f"{N}x{K} M={M}")
+    plain = [m for m in range(M) if m not in (1, M - 1)]
+    assert np.array_equal(run(ctx, 2, raw, N, K, base)[plain], y[plain])

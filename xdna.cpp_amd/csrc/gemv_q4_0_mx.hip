@@ -11,7 +11,13 @@
 // planes, hi = f16(x s) and lo = f16(x s - hi), s the power of two that puts
 // the largest |x| of the wavefront's part of the row in [2^14, 2^15): x to
 // 2^-22 of itself, or 2^-39 of that largest value.  Codes are exact, products
-// exact in f32; a block's f32 sums are scaled by its d and added in f32.
+// exact in f32; a block's f32 sums are scaled by its d and added in f32.  An
+// activation with a block whose largest value is more than 2^18 below that of the
+// wavefront's part is wide (the fixed point of the dot-unit forms, with a scale
+// per block, held such a block to 2^-20): after its tiles the workgroup sums wide
+// activations in f32 from their values as they are.  One comparison per lane
+// tells that there is none.  (us at 8192x8192 M = 8 with none, one and all wide
+// 19.7, 40, 90; the comparison costs 0.3.)
 //
 // Work split.  A workgroup of 8 wavefronts owns tiles of 16 weight rows and
 // splits K: wavefront v takes QN quads of 4 blocks.  Lane (n, g) = (lane & 15,
@@ -28,8 +34,8 @@
 // What bounds it.  VALU issue: about 85 instructions per quad and tile and 78
 // per quad to stage the activations, which every workgroup does for itself, so
 // long rows with few tiles per workgroup spend most of their time staging.
-// us per call on MI355X, dot-unit forms -> here: M = 8 8192x8192 25.9 -> 19.3,
-// 4096x4096 11.9 -> 8.2, 17408x5120 42.9 -> 19.7, 151936x2048 73.7 -> 49.
+// us per call on MI355X, dot-unit forms -> here: M = 8 8192x8192 25.9 -> 19.7,
+// 4096x4096 11.9 -> 8.2, 17408x5120 42.9 -> 19.9, 151936x2048 73.7 -> 50.
 #include "internal.h"
 #include "kq_device.h"
 #include "q4_0_layout.h"
@@ -49,6 +55,7 @@ constexpr int kQxThreads = 64 * kQxWaves;
 constexpr int kQxRows = 16;     // weight rows per tile
 constexpr int kQxAct = 8;       // activations per launch
 constexpr int kQxMaxQuads = 8;  // quads of blocks per wavefront and launch
+constexpr float kQxBelow = 0.0625f;  // largest scaled value from which on a block's planes hold it to 2^-21
 
 struct QxArgs {
     const uint8_t *W;
@@ -122,10 +129,103 @@ __device__ __forceinline__ uint32_t qx_from(f16x2 own, f16x2 other) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(__builtin_bit_cast(int, own),
                                                              __builtin_bit_cast(int, other), 0x128, 0xF, BANKS, false));
 }
+__device__ __forceinline__ float qx_max4(const float4 &f) {
+    return fmaxf(fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fabsf(f.z)), fabsf(f.w));
+}
+// over the 8 lanes of an activation: the two planes' (row_ror:8) and the lane groups
+__device__ __forceinline__ float qx_row_max(float v) {
+    v = fmaxf(v, dpp_mov<0x128>(v));
+    v = fmaxf(v, __shfl_xor(v, 16));
+    return fmaxf(v, __shfl_xor(v, 32));
+}
+__device__ __forceinline__ uint32_t qx_row_or(uint32_t v) {
+    v |= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x128, 0xF, 0xF, false));
+    v |= __shfl_xor(v, 16);
+    return v | __shfl_xor(v, 32);
+}
+
+// A weight row of a tile: block b of it in lane group b & 3 (the lane's 16 code
+// bytes and d).  The tile's rows are one buffer, empty past the last tile and
+// where `in` is false (readfirstlane: left alone, the compiler computes the
+// descriptor in vector registers and loops over its values).
+__device__ __forceinline__ void qx_load(const QxArgs &a, int tile, bool in, uint32_t b, int col, u32x4 &q, uint32_t &d) {
+    const int rows = __builtin_amdgcn_readfirstlane(tile < a.tiles && in ? min(a.N - tile * kQxRows, kQxRows) : 0);
+    const int at = __builtin_amdgcn_readfirstlane(rows > 0 ? tile : 0);
+    const uint8_t *base = a.W + static_cast<int64_t>(at) * (kQxRows * a.row_bytes);
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(base), 0, static_cast<uint32_t>(rows * a.row_bytes), kBufferWord3);
+    const uint32_t F = static_cast<uint32_t>(a.B) >> 6;
+    const uint32_t slot = b < 64 * F ? (b & 63) * F + (b >> 6) : b;  // q4_0_d_slot
+    const uint32_t row = static_cast<uint32_t>(col) * static_cast<uint32_t>(a.row_bytes);
+    q = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(row + 16 * b), 0, kNonTemporal);
+    d = __builtin_amdgcn_raw_buffer_load_b16(rsrc, static_cast<int>(row + 16 * static_cast<uint32_t>(a.B) + 2 * slot), 0, 0);
+}
+
+// The activations of `wide`, over quads [qw, qw + n) of this wavefront, in f32:
+// each lane its block of its weight row.  red: 8 wavefronts x 8 activations x 16
+// rows.  Called by the whole workgroup with the same `wide`.
+__device__ __forceinline__ void qx_wide(const QxArgs &a, uint32_t wide, int qw, int n, int wave, int lane,
+                                        float (*red)[kQxAct][kQxRows]) {
+    const int col = lane & 15, g = lane >> 4;
+    for (int tile = blockIdx.x; tile < a.tiles; tile += static_cast<int>(gridDim.x)) {
+        float acc[kQxAct] = {};
+#pragma clang loop unroll(disable)
+        for (int i = 0; i < n && qw + i < a.q1; ++i) {
+            const uint32_t b = 4u * static_cast<uint32_t>(qw + i) + g;
+            u32x4 q;
+            uint32_t dh;
+            qx_load(a, tile, true, b, col, q, dh);
+            float w[32];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const f16x8 o = qx_operand(q[k]);  // values 0, 2, 1, 3 of the low nibbles, then of the high ones
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    w[16 * t + 4 * k] = static_cast<float>(o[4 * t]);
+                    w[16 * t + 4 * k + 2] = static_cast<float>(o[4 * t + 1]);
+                    w[16 * t + 4 * k + 1] = static_cast<float>(o[4 * t + 2]);
+                    w[16 * t + 4 * k + 3] = static_cast<float>(o[4 * t + 3]);
+                }
+            }
+            const float d = half_f(dh);
+#pragma unroll
+            for (int m = 0; m < kQxAct; ++m) {
+                if (!(wide >> m & 1)) continue;
+                const float *x = a.x + m * a.x_stride + 32 * static_cast<int64_t>(b);
+                float s = 0.f;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const float4 v = qx_load4(x + 4 * k);
+                    s += fmaf(w[4 * k], v.x, w[4 * k + 1] * v.y) + fmaf(w[4 * k + 2], v.z, w[4 * k + 3] * v.w);
+                }
+                acc[m] = fmaf(d, s, acc[m]);
+            }
+        }
+        __syncthreads();  // the last readers of red
+#pragma unroll
+        for (int m = 0; m < kQxAct; ++m) {
+            float v = acc[m];
+            v += __shfl_xor(v, 16);
+            v += __shfl_xor(v, 32);
+            if (g == 0) red[wave][m][col] = v;
+        }
+        __syncthreads();
+        const int m = 2 * (wave & 3) + (lane >> 5), r = lane & 31;
+        if (wave < 4 && r < kQxRows && (wide >> m & 1) && tile * kQxRows + r < a.N) {
+            float v = 0.f;
+#pragma unroll
+            for (int k = 0; k < kQxWaves; ++k) v += red[k][m][r];
+            float *y = a.y + m * a.y_stride + tile * kQxRows + r;
+            *y = a.add ? *y + v : v;
+        }
+    }
+}
+
 template <int QN>
 __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     __shared__ f32x4 part[2][kQxWaves][64];
     __shared__ float unit[kQxWaves][kQxAct];
+    __shared__ uint32_t wides[kQxWaves];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int col = lane & 15, g = lane >> 4;
@@ -148,23 +248,8 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     // 2. the first tile's weights
     u32x4 wq[QN];
     uint32_t wd[QN];
-    const uint32_t F = static_cast<uint32_t>(a.B) >> 6;
     auto load = [&](int i, int tile) {
-        // the tile's rows as one buffer, empty past the last tile and past the
-        // launch's quads (readfirstlane: left alone, the compiler computes the
-        // descriptor in vector registers and loops over its values)
-        const int rows = __builtin_amdgcn_readfirstlane(
-            tile < a.tiles && qw + i < a.q1 ? min(a.N - tile * kQxRows, kQxRows) : 0);
-        const int at = __builtin_amdgcn_readfirstlane(rows > 0 ? tile : 0);
-        const uint8_t *base = a.W + static_cast<int64_t>(at) * (kQxRows * a.row_bytes);
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint8_t *>(base), 0, static_cast<uint32_t>(rows * a.row_bytes), kBufferWord3);
-        const uint32_t b = 4u * static_cast<uint32_t>(qw + i) + g;
-        const uint32_t slot = b < 64 * F ? (b & 63) * F + (b >> 6) : b;  // q4_0_d_slot
-        const uint32_t row = static_cast<uint32_t>(col) * static_cast<uint32_t>(a.row_bytes);
-        wq[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(row + 16 * b), 0, kNonTemporal);
-        wd[i] = __builtin_amdgcn_raw_buffer_load_b16(
-            rsrc, static_cast<int>(row + 16 * static_cast<uint32_t>(a.B) + 2 * slot), 0, 0);
+        qx_load(a, tile, qw + i < a.q1, 4u * static_cast<uint32_t>(qw + i) + g, col, wq[i], wd[i]);
     };
     int tile = blockIdx.x;
 #pragma unroll
@@ -172,22 +257,41 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     __builtin_amdgcn_sched_barrier(0);
 
     // 3. the activations' operands
-    float mxe[4] = {0.f, 0.f, 0.f, 0.f};
+    float mxe[2] = {0.f, 0.f}, mn = __builtin_inff();  // mn: smallest of the lane's quarters of blocks
 #pragma unroll
     for (int i = 0; i < QN; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            mxe[e] = fmaxf(fmaxf(mxe[e], fabsf(f[i][e].x)), fabsf(f[i][e].y));
-            mxe[e] = fmaxf(fmaxf(mxe[e], fabsf(f[i][e].z)), fabsf(f[i][e].w));
+        for (int e = 0; e < 2; ++e) {
+            const float q0 = qx_max4(f[i][2 * e]), q1 = qx_max4(f[i][2 * e + 1]);
+            mxe[e] = fmaxf(fmaxf(mxe[e], q0), q1);
+            mn = fminf(fminf(mn, q0), q1);
         }
-    float mx = fmaxf(fmaxf(mxe[0], mxe[1]), fmaxf(mxe[2], mxe[3]));
-    mx = fmaxf(mx, dpp_mov<0x128>(mx));  // row_ror:8, the row's other plane
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float mx = qx_row_max(fmaxf(mxe[0], mxe[1]));
     // s = 2^(14 - E) for mx in [2^E, 2^(E+1)), E >= -110, and 1 / s
     const int ex = min(max(static_cast<int>(__builtin_bit_cast(uint32_t, mx) >> 23), 17), 254);
     const float s = __builtin_bit_cast(float, static_cast<uint32_t>(268 - ex) << 23);
     if (lane < kQxAct) unit[wave][lane] = __builtin_bit_cast(float, static_cast<uint32_t>(ex - 14) << 23);
+    uint32_t wide = 0;  // of this wavefront's part
+    if (!__all(mn * s >= kQxBelow)) {
+        // block by block: bits of the lane's quarters that are large enough, and
+        // that are not 0 (the smallest scale takes what it has)
+        const float below = ex > 17 ? kQxBelow : 0.f;
+        uint32_t near = 0, some = 0;
+#pragma unroll
+        for (int i = 0; i < QN; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float4 v = f[i][e];
+                asm volatile("" : "+v"(v.x));  // its maximum anew: kept from above, all would be live here
+                const float q = qx_max4(v);
+                near |= q * s >= below ? 1u << (4 * i + e) : 0u;
+                some |= q > 0.f ? 1u << (4 * i + e) : 0u;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        const uint32_t far = qx_row_or(some) & ~qx_row_or(near);
+        wide = static_cast<uint32_t>(__ballot(far != 0)) & 0xFF;
+    }
+    if (lane == 0) wides[wave] = wide;
     f16x8 x[QN][4];
 #pragma unroll
     for (int i = 0; i < QN; ++i) {
@@ -204,6 +308,21 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     }
     // result row 4 g + k of this wavefront is activation (4 g + k) & 7
     const f32x4 u = *reinterpret_cast<const f32x4 *>(&unit[wave][4 * (g & 1)]);
+
+    // the workgroup's wide activations: an adding launch leaves theirs out below,
+    // the others overwrite them
+    auto wide_all = [&] {
+        uint32_t v = wides[threadIdx.x & (kQxWaves - 1)];
+        v |= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, false));
+        v |= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false));
+        v |= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xF, 0xF, false));
+        return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))) & ((1u << a.M) - 1);
+    };
+    wide = 0;
+    if (a.add) {
+        __syncthreads();
+        wide = wide_all();
+    }
 
     // 4. tiles
     for (int par = 0; tile < a.tiles; par ^= 1) {
@@ -238,11 +357,17 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
         sum += quad_x1_f(sum);
         sum += quad_x2_f(sum);
         const int n = tile * kQxRows + on;
-        if (w == 0 && om < a.M && n < a.N) {
+        if (w == 0 && om < a.M && n < a.N && !(wide >> om & 1)) {
             float *y = a.y + om * a.y_stride + n;
             *y = a.add ? *y + sum : sum;
         }
         tile = next;
+    }
+    wide = wide_all();  // a workgroup has a tile, so a barrier has passed
+    if (wide) {
+        int l = threadIdx.x & 63;
+        asm volatile("" : "+v"(l));  // nothing stays in registers for this over the tiles
+        qx_wide(a, wide, qw, QN, wave, l, reinterpret_cast<float(*)[kQxAct][kQxRows]>(part));
     }
 }
 
