@@ -224,7 +224,7 @@ __device__ __forceinline__ void qx_wide(const QxArgs &a, uint32_t wide, int qw, 
 template <int QN>
 __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     __shared__ f32x4 part[2][kQxWaves][64];
-    __shared__ float unit[kQxWaves][kQxAct];
+    __shared__ f32x4 unit[kQxWaves][kQxAct / 4];
     __shared__ uint32_t wides[kQxWaves];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -270,7 +270,8 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     // s = 2^(14 - E) for mx in [2^E, 2^(E+1)), E >= -110, and 1 / s
     const int ex = min(max(static_cast<int>(__builtin_bit_cast(uint32_t, mx) >> 23), 17), 254);
     const float s = __builtin_bit_cast(float, static_cast<uint32_t>(268 - ex) << 23);
-    if (lane < kQxAct) unit[wave][lane] = __builtin_bit_cast(float, static_cast<uint32_t>(ex - 14) << 23);
+    if (lane < kQxAct)
+        reinterpret_cast<float *>(unit[wave])[lane] = __builtin_bit_cast(float, static_cast<uint32_t>(ex - 14) << 23);
     uint32_t wide = 0;  // of this wavefront's part
     if (!__all(mn * s >= kQxBelow)) {
         // block by block: bits of the lane's quarters that are large enough, and
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
         }
     }
     // result row 4 g + k of this wavefront is activation (4 g + k) & 7
-    const f32x4 u = *reinterpret_cast<const f32x4 *>(&unit[wave][4 * (g & 1)]);
+    const f32x4 u = unit[wave][g & 1];
 
     // the workgroup's wide activations: an adding launch leaves theirs out below,
     // the others overwrite them
