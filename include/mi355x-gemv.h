@@ -82,7 +82,9 @@ MI355X_API const char *mi355x_last_error(void);
  * (a hipError_t value): MI355X_EHIP (MI355X_ENOMEM for hipErrorOutOfMemory)
  * with mi355x_last_error() = "<entry>: <hipErrorName> (<hipErrorString>)
  * [injected]".  One fault at a time, process-wide, disarmed once it fired;
- * entry NULL disarms.  The environment variable
+ * entry NULL disarms.  The name "mi355x_ctx_workspace" (not reached by "*")
+ * instead makes mi355x_ctx_create find no room for the workspace of batched
+ * calls, which is no error.  The environment variable
  * MI355X_INJECT_FAULT="<entry>:<hip_error>[:<skip>]" arms one at first use
  * of the library. */
 MI355X_API int mi355x_inject_fault(const char *entry, int hip_error, int skip);
@@ -290,8 +292,9 @@ MI355X_API int mi355x_gemv_bf16(mi355x_ctx *ctx, int type, const void *W, int64_
  * sum a codebook type in f32) run on the matrix cores, up to 512 per pass over
  * the weights: activations as two f16 planes (22 bits), products exact, f32
  * sums (one launch that splits the activations into the context's 64 MiB
- * workspace, allocated with the context and freed with it, one product
- * launch, and one that adds the partial sums where K is split; IQ3_XXS and
+ * workspace, allocated with the context and freed with it -- a context created
+ * where the device has no room for it runs such calls in the other forms --, one
+ * product launch, and one that adds the partial sums where K is split; IQ3_XXS and
  * IQ2_S with grids of magnitudes up to 66).  A few activations (2 to 8, as
  * many as fit the LDS) of the other types run in one launch with the one-row
  * kernels' digit arithmetic on the integer matrix cores, where those kernels
@@ -326,9 +329,9 @@ MI355X_API int mi355x_gemv_batched(mi355x_ctx *ctx, int type, const void *W, int
  * one device shares that scratch: calls that overlap on one device (two
  * streams or contexts of the same device) race.  Nothing else allocates:
  * K/IQ weights need 16-byte aligned activation rows (x and x_stride a
- * multiple of 4 floats), IQ3_XXS / IQ2_S need their grid already on the
- * context (one mi355x_gemv of the type first); otherwise MI355X_EINVAL /
- * MI355X_EUNSUPPORTED with a message. */
+ * multiple of 4 floats; some forms would copy others), IQ3_XXS / IQ2_S need
+ * their grid already on the context (one mi355x_gemv of the type first);
+ * otherwise MI355X_EINVAL / MI355X_EUNSUPPORTED with a message. */
 #define MI355X_NOALLOC_SCRATCH_BYTES 344064
 MI355X_API int mi355x_gemv_batched_noalloc(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
                                            const float *x, int64_t x_stride, float *y, int64_t y_stride,

@@ -208,6 +208,21 @@ void read_fault_env() {
     arm_fault(spec.substr(0, c1).c_str(), error, skip);
 }
 
+// Whether a fault is armed under exactly this name ("*" means entry points);
+// disarms it.
+bool take_fault(const char *name) {
+    std::call_once(g_fault_env_once, read_fault_env);
+    if (!g_fault.armed.load(std::memory_order_relaxed)) return false;
+    std::lock_guard<std::mutex> lk(g_fault.mu);
+    if (!g_fault.armed.load() || g_fault.entry != name) return false;
+    if (g_fault.skip > 0) {
+        --g_fault.skip;
+        return false;
+    }
+    g_fault.armed.store(false);
+    return true;
+}
+
 }  // namespace
 
 int device_gate(const mi355x_ctx *ctx, const char *entry) {
@@ -408,7 +423,7 @@ int mi355x_ctx_create(int device, mi355x_ctx **out) {
         return set_error(rc, msg);
     }
     // batched calls do without it if the device has no room
-    if (hipMalloc(&ctx->gemm_buf, kGemmWorkspace) != hipSuccess) {
+    if (take_fault("mi355x_ctx_workspace") || hipMalloc(&ctx->gemm_buf, kGemmWorkspace) != hipSuccess) {
         (void)hipGetLastError();
         ctx->gemm_buf = nullptr;
     }
@@ -918,9 +933,10 @@ int gemv_batched(mi355x_ctx *ctx, int type, const void *W, int64_t N, int64_t K,
         return set_error(MI355X_EINVAL, std::string(who) + ": strides smaller than a row");
     if (noalloc && ctx && M > 0 && N > 0) {
         if (!ctx->scratch) return set_error(MI355X_EUNSUPPORTED, std::string(who) + ": no static scratch on the device");
-        // the K/IQ kernels copy unaligned activations into a context buffer,
-        // and IQ3_XXS / IQ2_S grids reach a context on its first such GEMV:
-        // both would allocate
+        // some K/IQ kernels (GGML_Q8, forms that an option selects) copy
+        // unaligned activations into a context buffer, so unaligned rows are
+        // refused whichever form would run; IQ3_XXS / IQ2_S grids reach a
+        // context on its first such GEMV: both would allocate
         if (type != MI355X_TYPE_Q4_0 &&
             ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (M > 1 && (x_stride & 3) != 0)))
             return set_error(MI355X_EINVAL, std::string(who) +
