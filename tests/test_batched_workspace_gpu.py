@@ -12,8 +12,9 @@ from tolerance import check_f32_sum, product64
 pytestmark = pytest.mark.gpu
 
 # 64 MiB hold 248 rows of 65536 values (passes of 160 and 140 here) and 512 rows
-# of 30208 with 2 MiB left for partial sums (4 segments of N = 256, M = 512)
-SIZES = [("Q4_K", 40, 65536, 300), ("Q6_K", 256, 30208, 512), ("IQ3_S", 33, 65536, 260)]
+# of 30208 with 2 MiB left for partial sums (4 segments of N = 256, M = 512);
+# rows past 124 superblocks in passes of 32 to the end
+SIZES = [("Q4_K", 40, 65536, 300), ("Q6_K", 256, 30208, 512), ("IQ3_S", 33, 65536, 260), ("Q3_K", 70, 262144, 70)]
 
 
 @pytest.mark.parametrize("name,N,K,M", SIZES)

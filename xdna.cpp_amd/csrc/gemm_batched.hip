@@ -1058,8 +1058,9 @@ __global__ __launch_bounds__(kGmThreads, 2) void gemm_kernel(GemmArgs a) {
     }
 }
 
-// y = partial 0 + partial 1 + ..., in segment order, in Sum (f64 for the FINE
-// kernels' partials, which costs 1.8 us more at 4 x 512 x 4096)
+// y = partial 0 + partial 1 + ..., in segment order, in Sum (f64, which costs 1.8
+// us more at 4 x 512 x 4096, for the FINE kernels' partials and for more than 64,
+// whose f32 chain loses: 5e-7 of an output's deviation with 512)
 template <class Sum>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float *part, int64_t seg_stride, int nseg, int M,
                                                           int64_t N, float *y, int64_t y_stride) {
@@ -1214,7 +1215,7 @@ int launch_gemm_batched(mi355x_ctx *ctx, const GemvArgs &a, int64_t x_stride, in
                            ctx->stream, g);
         MI355X_HIP(hipGetLastError());
         if (g.nseg > 1) {
-            hipLaunchKernelGGL(fine ? gemm_reduce_kernel<double> : gemm_reduce_kernel<float>,
+            hipLaunchKernelGGL(fine || g.nseg > 64 ? gemm_reduce_kernel<double> : gemm_reduce_kernel<float>,
                                dim3(static_cast<unsigned>((a.N + 255) / 256), std::min(M, 64)),
                                dim3(256), 0, ctx->stream, partial, g.seg_stride, g.nseg, M, a.N, y, y_stride);
             MI355X_HIP(hipGetLastError());
