@@ -7,6 +7,7 @@ import pytest
 
 import mi355x
 import synth
+from tolerance import DIGIT_SUM, check_sum, product64
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +83,22 @@ def test_digits_q4_0_long_rows_stay_refused(ctx):
     finally:
         for b in (w, x, y):
             b.free()
+
+
+@pytest.mark.parametrize("name,N,K", [("Q4_0", 300, 2048), ("Q4_0", 70, 8192), ("Q4_K", 300, 2048), ("Q6_K", 64, 8448),
+                                      ("IQ3_S", 300, 2048), ("IQ3_S", 4100, 2048), ("IQ4_XS", 64, 4096)])
+def test_output_across_batch_sizes(ctx, oracle, name, N, K):
+    """The same activation alone, among 4, 9, 21 and 40: the arithmetic depends on
+    the number (fixed point per 32 values of 20 bits for Q4_0 and 16 for the other
+    types, or two f16 planes, or f32), and each stays within its bound."""
+    t = 2 if name == "Q4_0" else KQ[name]
+    xs = rows(K, 40)
+    w = ctx.resident(t, synth.random_q4_0(N, K, 5) if t == 2 else synth.random_blocks(t, N, K, 5), N, K)
+    try:
+        ys = [ctx.gemv(w, xs[0])] + [ctx.gemv_batched(w, xs[:M])[0] for M in (4, 9, 21, 40)]
+        raw = w.raw_bytes()
+    finally:
+        w.free()
+    ref, norms = product64(oracle, t, raw, N, K, xs[:1])
+    for y in ys:
+        check_sum(y[None], ref, norms, xs[:1], DIGIT_SUM / 16 if t == 2 else DIGIT_SUM, name)

@@ -1,5 +1,5 @@
 """Matrix-core batched GEMV (mi355x_gemv_batched with many activations) on the
-GPU against the CPU oracle: every weight type, sizes around the tiles (256
+GPU against the CPU oracle and 64 bits: every weight type, sizes around the tiles (256
 weight rows per workgroup, 64 per wavefront, 32 or 64 activations per tile,
 256-value superblocks, K segments), strides and unaligned rows, extreme
 activation scales, and the allocation-free form, which must give the same
@@ -9,7 +9,7 @@ import pytest
 
 import mi355x
 import synth
-from tolerance import check_gemv
+from tolerance import F32_SUM, check_gemv, check_sum, product64
 
 pytestmark = pytest.mark.gpu
 
@@ -39,8 +39,11 @@ def weights(t, N, K, seed):
     return synth.random_q4_0(N, K, seed) if t == 2 else synth.random_blocks(t, N, K, seed)
 
 
-def check(oracle, t, raw, N, K, xs, y, what, grid=None):
+def check(oracle, t, raw, N, K, xs, y, what, grid=None, bound=None):
+    """Against the oracle, and against 64 bits within bound * ||w|| * rms(x)."""
     grid = GRIDS.get(t) if grid is None else grid
+    if bound:
+        check_sum(y, *product64(oracle, t, raw, N, K, xs, grid), xs, bound, what)
     norms = oracle.row_norms(t, raw, N, K, grid=grid)
     for m in range(xs.shape[0]):
         check_gemv(y[m], oracle.gemv(t, raw, N, K, xs[m], grid=grid), norms, xs[m], f"{what} activation {m}")
@@ -67,7 +70,7 @@ def test_gemm_matches_oracle(ctx, oracle, name, N, K, M):
     t = TYPES[name]
     raw = weights(t, N, K, N + K)
     xs = np.stack([synth.activations(K, seed=100 + m) for m in range(M)])
-    check(oracle, t, raw, N, K, xs, run(ctx, t, raw, N, K, xs), f"{name} {N}x{K} M={M}")
+    check(oracle, t, raw, N, K, xs, run(ctx, t, raw, N, K, xs), f"{name} {N}x{K} M={M}", bound=F32_SUM)
 
 
 def test_gemm_q4_0_partial_superblock(ctx, oracle):
@@ -75,7 +78,7 @@ def test_gemm_q4_0_partial_superblock(ctx, oracle):
     for N, K in ((70, 64), (300, 2048 + 192), (33, 4416)):
         raw = synth.random_q4_0(N, K, 3)
         xs = np.stack([synth.activations(K, seed=m) for m in range(20)])
-        check(oracle, 2, raw, N, K, xs, run(ctx, 2, raw, N, K, xs), f"Q4_0 {N}x{K}")
+        check(oracle, 2, raw, N, K, xs, run(ctx, 2, raw, N, K, xs), f"Q4_0 {N}x{K}", bound=F32_SUM)
 
 
 @pytest.mark.parametrize("name", ["Q4_0", "Q4_K", "IQ3_S"])
@@ -83,7 +86,7 @@ def test_gemm_more_rows_than_one_pass(ctx, oracle, name):
     t, N, K, M = TYPES[name], 130, 512, 520
     raw = weights(t, N, K, 4)
     xs = np.stack([synth.activations(K, seed=m) for m in range(M)])
-    check(oracle, t, raw, N, K, xs, run(ctx, t, raw, N, K, xs), f"{name} M={M}")
+    check(oracle, t, raw, N, K, xs, run(ctx, t, raw, N, K, xs), f"{name} M={M}", bound=F32_SUM)
 
 
 @pytest.mark.parametrize("name", list(TYPES))
@@ -125,7 +128,7 @@ def test_gemm_activation_scales_and_nonfinite(ctx, oracle, name):
     y = run(ctx, t, raw, N, K, xs)
     assert np.all(y[3] == 0.0)
     rows = [m for m in range(M) if m != 3]
-    check(oracle, t, raw, N, K, xs[rows], y[rows], name)
+    check(oracle, t, raw, N, K, xs[rows], y[rows], name, bound=F32_SUM)
     bad = xs.copy()
     bad[7, 300] = np.inf
     bad[8, 5] = np.nan

@@ -9,6 +9,7 @@ import pytest
 import mi355x
 import synth
 from test_gemm_batched_gpu import TYPES, check, install_grids, run, weights  # noqa: F401 (fixture)
+from tolerance import DIGIT_SUM
 
 pytestmark = pytest.mark.gpu
 
@@ -35,7 +36,7 @@ def test_few_activations_match_oracle(ctx, oracle, name, N, K, M):
         ctx.set_option(mi355x.OPT_VARIANT, mi355x.VARIANT_AUTO)
     rows = np.unique(np.concatenate([np.arange(min(N, 64)), np.arange(max(0, N - 64), N)]))
     sub = raw.reshape(N, -1)[rows]
-    check(oracle, t, sub, len(rows), K, xs, y[:, rows], f"{name} {N}x{K} M={M}")
+    check(oracle, t, sub, len(rows), K, xs, y[:, rows], f"{name} {N}x{K} M={M}", bound=DIGIT_SUM)
     if (t not in (14, 11, 18, 21, 22) or K <= 8192) and (t != 22 or K <= 4096):  # else two one-row launches
         assert np.array_equal(one, y[[M - 1, 0]])
 

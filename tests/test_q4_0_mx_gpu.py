@@ -1,5 +1,5 @@
 """mi355x_gemv_batched with a few Q4_0 activations on the matrix cores (one
-launch, activations as two f16 planes) on the GPU against the CPU oracle:
+launch, activations as two f16 planes) on the GPU against the CPU oracle and 64 bits:
 sizes around the 16-row tiles, the 4-block quads of a wavefront and the
 8192 values of a launch, strides and unaligned rows, more than one pass, the
 allocation-free form, and rows of very different scales."""
@@ -9,6 +9,7 @@ import pytest
 import mi355x
 import synth
 from test_gemm_batched_gpu import check, run, weights
+from tolerance import F32_SUM
 
 pytestmark = pytest.mark.gpu
 
@@ -29,7 +30,7 @@ def test_few_activations_match_oracle(ctx, oracle, N, K, M):
     xs = np.stack([synth.activations(K, seed=100 + m) for m in range(M)])
     y = run(ctx, 2, raw, N, K, xs)
     rows = some_rows(N)
-    check(oracle, 2, raw.reshape(N, -1)[rows], len(rows), K, xs, y[:, rows], f"{N}x{K} M={M}")
+    check(oracle, 2, raw.reshape(N, -1)[rows], len(rows), K, xs, y[:, rows], f"{N}x{K} M={M}", bound=F32_SUM)
     # an activation's result does not depend on the others
     assert np.array_equal(run(ctx, 2, raw, N, K, xs[::-1].copy())[::-1], y)
 
@@ -63,5 +64,11 @@ def test_few_activations_scales(ctx, oracle):
     step = np.where(np.arange(K) < K // 2, 2.0 ** -20, 1.0).astype(np.float32)
     xs = np.stack([x * np.float32(1e-30), x, x * np.float32(1e30), np.zeros_like(x), x * step])
     y = run(ctx, 2, raw, N, K, xs)
-    check(oracle, 2, raw, N, K, xs, y, "scales")
+    check(oracle, 2, raw, N, K, xs, y, "scales", bound=F32_SUM)
     assert not y[3].any()
+    # the small part on its own: the weights of the other are 0
+    small = raw.reshape(N, K // 32, 18).copy()
+    small[:, K // 64:, :2] = 0
+    alone = np.where(np.arange(K) < K // 2, xs[4:], 0.0)
+    check(oracle, 2, small.reshape(N, -1), N, K, alone, run(ctx, 2, small.reshape(N, -1), N, K, xs)[4:], "small part",
+          bound=F32_SUM)
