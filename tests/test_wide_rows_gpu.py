@@ -62,6 +62,9 @@ def test_few_wide_q4_0_rows(ctx, oracle, N, K, M):
     base = np.stack([synth.activations(K, seed=50 + m) for m in range(M)])
     base[:, :32] = base[:, -32:] = 0
     base[0, 64:128] = 0  # blocks of zeros are not small
+    base[1, np.arange(K) % 4 != K % 7 % 4] = 0  # one value in four, and blocks of a single one
+    base[1, 128:192] = 0
+    base[1, 131] = 1.0
     xs = base.copy()
     xs[1, 3] = 2.0 ** 24
     xs[M - 1] *= 2.0 ** -60

@@ -15,9 +15,10 @@
 // activation with a block whose largest value is more than 2^18 below that of the
 // wavefront's part is wide (the fixed point of the dot-unit forms, with a scale
 // per block, held such a block to 2^-20): after its tiles the workgroup sums wide
-// activations in f32 from their values as they are.  One comparison per lane
-// tells that there is none.  (us at 8192x8192 M = 8 with none, one and all wide
-// 19.7, 40, 90; the comparison costs 0.3.)
+// activations in f32 from their values as they are.  The lanes compare the least
+// that they saw of each activation while they stage it; only where that is small
+// does the workgroup read the activations again to tell.  (us at 8192x8192 M = 8
+// with none, one and all wide 19.8, 48, 95, without the comparison 19.3.)
 //
 // Work split.  A workgroup of 8 wavefronts owns tiles of 16 weight rows and
 // splits K: wavefront v takes QN quads of 4 blocks.  Lane (n, g) = (lane & 15,
@@ -34,8 +35,8 @@
 // What bounds it.  VALU issue: about 85 instructions per quad and tile and 78
 // per quad to stage the activations, which every workgroup does for itself, so
 // long rows with few tiles per workgroup spend most of their time staging.
-// us per call on MI355X, dot-unit forms -> here: M = 8 8192x8192 25.9 -> 19.7,
-// 4096x4096 11.9 -> 8.2, 17408x5120 42.9 -> 19.9, 151936x2048 73.7 -> 50.
+// us per call on MI355X, dot-unit forms -> here: M = 8 8192x8192 25.9 -> 19.8,
+// 4096x4096 11.9 -> 8.3, 17408x5120 42.9 -> 20.0, 151936x2048 73.7 -> 50.
 #include "internal.h"
 #include "kq_device.h"
 #include "q4_0_layout.h"
@@ -143,6 +144,13 @@ __device__ __forceinline__ uint32_t qx_row_or(uint32_t v) {
     v |= __shfl_xor(v, 16);
     return v | __shfl_xor(v, 32);
 }
+// s = 2^(14 - E) for mx in [2^E, 2^(E+1)), E >= -110, and unit = 1 / s
+constexpr float kQxUnitMin = 0x1p-124f;
+__device__ __forceinline__ float qx_scale(float mx, float &unit) {
+    const int ex = min(max(static_cast<int>(__builtin_bit_cast(uint32_t, mx) >> 23), 17), 254);
+    unit = __builtin_bit_cast(float, static_cast<uint32_t>(ex - 14) << 23);
+    return __builtin_bit_cast(float, static_cast<uint32_t>(268 - ex) << 23);
+}
 
 // A weight row of a tile: block b of it in lane group b & 3 (the lane's 16 code
 // bytes and d).  The tile's rows are one buffer, empty past the last tile and
@@ -161,17 +169,36 @@ __device__ __forceinline__ void qx_load(const QxArgs &a, int tile, bool in, uint
     d = __builtin_amdgcn_raw_buffer_load_b16(rsrc, static_cast<int>(row + 16 * static_cast<uint32_t>(a.B) + 2 * slot), 0, 0);
 }
 
-// The activations of `wide`, over quads [qw, qw + n) of this wavefront, in f32:
+// The activations (bits) of which quads [qw, qw + n), n <= 8, hold a block that
+// the planes lose, `unit` the lane's activation's: read again, as this is seldom
+// asked (parts with such blocks, or with zeros).
+__device__ __forceinline__ uint32_t qx_lost(const QxArgs &a, int qw, int n, int lane, float unit) {
+    const int m = lane & 7, g = lane >> 4, plane = (lane >> 3) & 1;
+    const float *x = a.x + min(m, a.M - 1) * a.x_stride + 4 * g + 16 * plane;
+    // the smallest scale takes what it has
+    const float below = unit > kQxUnitMin ? kQxBelow * unit : 0.f;
+    // bits of the lane's quarters that are large enough, and that are not 0
+    uint32_t near = 0, some = 0;
+#pragma unroll 16
+    for (int k = 0; k < 4 * n; ++k) {
+        const float q = qx_max4(qx_load4(x + 32 * static_cast<int64_t>(min(4 * qw + k, 4 * a.q1 - 1))));
+        near |= static_cast<uint32_t>(q >= below) << k;
+        some |= static_cast<uint32_t>(q > 0.f) << k;
+    }
+    return static_cast<uint32_t>(__ballot((qx_row_or(some) & ~qx_row_or(near)) != 0)) & 0xFF;
+}
+
+// The activations of `wide` over the whole row so far, quads [0, q1), in f32:
 // each lane its block of its weight row.  red: 8 wavefronts x 8 activations x 16
-// rows.  Called by the whole workgroup with the same `wide`.
-__device__ __forceinline__ void qx_wide(const QxArgs &a, uint32_t wide, int qw, int n, int wave, int lane,
-                                        float (*red)[kQxAct][kQxRows]) {
+// rows.  Called by the whole workgroup with the same `wide`; replaces what the
+// tiles stored (and what the launch before did).
+__device__ __forceinline__ void qx_wide(const QxArgs &a, uint32_t wide, int wave, int lane, float (*red)[kQxAct][kQxRows]) {
     const int col = lane & 15, g = lane >> 4;
     for (int tile = blockIdx.x; tile < a.tiles; tile += static_cast<int>(gridDim.x)) {
         float acc[kQxAct] = {};
 #pragma clang loop unroll(disable)
-        for (int i = 0; i < n && qw + i < a.q1; ++i) {
-            const uint32_t b = 4u * static_cast<uint32_t>(qw + i) + g;
+        for (int qd = wave; qd < a.q1; qd += kQxWaves) {
+            const uint32_t b = 4u * static_cast<uint32_t>(qd) + g;
             u32x4 q;
             uint32_t dh;
             qx_load(a, tile, true, b, col, q, dh);
@@ -215,8 +242,7 @@ __device__ __forceinline__ void qx_wide(const QxArgs &a, uint32_t wide, int qw, 
             float v = 0.f;
 #pragma unroll
             for (int k = 0; k < kQxWaves; ++k) v += red[k][m][r];
-            float *y = a.y + m * a.y_stride + tile * kQxRows + r;
-            *y = a.add ? *y + v : v;
+            a.y[m * a.y_stride + tile * kQxRows + r] = v;
         }
     }
 }
@@ -225,7 +251,7 @@ template <int QN>
 __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     __shared__ f32x4 part[2][kQxWaves][64];
     __shared__ f32x4 unit[kQxWaves][kQxAct / 4];
-    __shared__ uint32_t wides[kQxWaves];
+    __shared__ uint32_t flags[kQxWaves];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int col = lane & 15, g = lane >> 4;
@@ -257,42 +283,25 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     __builtin_amdgcn_sched_barrier(0);
 
     // 3. the activations' operands
-    float mxe[2] = {0.f, 0.f}, mn = __builtin_inff();  // mn: smallest of the lane's quarters of blocks
+    // the largest value, and the smallest of the lane's quarters of blocks that is
+    // not 0 (its bits less 1, so that 0 is none)
+    float mxe[2] = {0.f, 0.f};
+    uint32_t mn = ~0u;
 #pragma unroll
     for (int i = 0; i < QN; ++i)
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const float q0 = qx_max4(f[i][2 * e]), q1 = qx_max4(f[i][2 * e + 1]);
             mxe[e] = fmaxf(fmaxf(mxe[e], q0), q1);
-            mn = fminf(fminf(mn, q0), q1);
+            mn = min(min(mn, __builtin_bit_cast(uint32_t, q0) - 1u), __builtin_bit_cast(uint32_t, q1) - 1u);
         }
     const float mx = qx_row_max(fmaxf(mxe[0], mxe[1]));
-    // s = 2^(14 - E) for mx in [2^E, 2^(E+1)), E >= -110, and 1 / s
-    const int ex = min(max(static_cast<int>(__builtin_bit_cast(uint32_t, mx) >> 23), 17), 254);
-    const float s = __builtin_bit_cast(float, static_cast<uint32_t>(268 - ex) << 23);
-    if (lane < kQxAct)
-        reinterpret_cast<float *>(unit[wave])[lane] = __builtin_bit_cast(float, static_cast<uint32_t>(ex - 14) << 23);
-    uint32_t wide = 0;  // of this wavefront's part
-    if (!__all(mn * s >= kQxBelow)) {
-        // block by block: bits of the lane's quarters that are large enough, and
-        // that are not 0 (the smallest scale takes what it has)
-        const float below = ex > 17 ? kQxBelow : 0.f;
-        uint32_t near = 0, some = 0;
-#pragma unroll
-        for (int i = 0; i < QN; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float4 v = f[i][e];
-                asm volatile("" : "+v"(v.x));  // its maximum anew: kept from above, all would be live here
-                const float q = qx_max4(v);
-                near |= q * s >= below ? 1u << (4 * i + e) : 0u;
-                some |= q > 0.f ? 1u << (4 * i + e) : 0u;
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        const uint32_t far = qx_row_or(some) & ~qx_row_or(near);
-        wide = static_cast<uint32_t>(__ballot(far != 0)) & 0xFF;
-    }
-    if (lane == 0) wides[wave] = wide;
+    float un;
+    const float s = qx_scale(mx, un);
+    if (lane < kQxAct) reinterpret_cast<float *>(unit[wave])[lane] = un;
+    // where each quarter is 0 or large enough, each block is
+    const bool suspect = !__all(mn + 1u >= __builtin_bit_cast(uint32_t, kQxBelow * un) || mn == ~0u);
+    if (lane == 0) flags[wave] = suspect;
     f16x8 x[QN][4];
 #pragma unroll
     for (int i = 0; i < QN; ++i) {
@@ -309,21 +318,6 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
     }
     // result row 4 g + k of this wavefront is activation (4 g + k) & 7
     const f32x4 u = unit[wave][g & 1];
-
-    // the workgroup's wide activations: an adding launch leaves theirs out below,
-    // the others overwrite them
-    auto wide_all = [&] {
-        uint32_t v = wides[threadIdx.x & (kQxWaves - 1)];
-        v |= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, false));
-        v |= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false));
-        v |= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x141, 0xF, 0xF, false));
-        return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))) & ((1u << a.M) - 1);
-    };
-    wide = 0;
-    if (a.add) {
-        __syncthreads();
-        wide = wide_all();
-    }
 
     // 4. tiles
     for (int par = 0; tile < a.tiles; par ^= 1) {
@@ -358,17 +352,25 @@ __global__ __launch_bounds__(kQxThreads) void gemv_q4_0_mx_kernel(QxArgs a) {
         sum += quad_x1_f(sum);
         sum += quad_x2_f(sum);
         const int n = tile * kQxRows + on;
-        if (w == 0 && om < a.M && n < a.N && !(wide >> om & 1)) {
+        if (w == 0 && om < a.M && n < a.N) {
             float *y = a.y + om * a.y_stride + n;
             *y = a.add ? *y + sum : sum;
         }
         tile = next;
     }
-    wide = wide_all();  // a workgroup has a tile, so a barrier has passed
-    if (wide) {
-        int l = threadIdx.x & 63;
-        asm volatile("" : "+v"(l));  // nothing stays in registers for this over the tiles
-        qx_wide(a, wide, qw, QN, wave, l, reinterpret_cast<float(*)[kQxAct][kQxRows]>(part));
+    // 5. wide activations (a workgroup has a tile, so a barrier has passed)
+    int l = threadIdx.x & 63;
+    asm volatile("" : "+v"(l));  // nothing stays in registers for this over the tiles
+    if (__builtin_expect(__any(flags[l & (kQxWaves - 1)] != 0), 0)) {
+        __syncthreads();  // every wavefront has read its flags
+        const uint32_t lost = qx_lost(a, qw, QN, l, reinterpret_cast<const float *>(unit[wave])[l & 7]);
+        if (l == 0) flags[wave] = lost;
+        __syncthreads();
+        uint32_t wide = 0;
+#pragma unroll
+        for (int k = 0; k < kQxWaves; ++k) wide |= flags[k];
+        wide = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(wide))) & ((1u << a.M) - 1);
+        if (wide) qx_wide(a, wide, wave, l, reinterpret_cast<float(*)[kQxAct][kQxRows]>(part));
     }
 }
 
