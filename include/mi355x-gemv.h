@@ -122,11 +122,16 @@ MI355X_API int mi355x_device_describe(int device, char *name, size_t name_len, c
  *       Q4_K, Q5_K and Q6_K, IQ4_XS rows of at most 8192 values, and
  *       IQ3_S/IQ3_XXS/IQ2_S rows of at most 8192 values with N >= 4096, one
  *       row per wavefront step; f32 activations for the rest: longer IQ rows
- *       and smaller IQ matrices),
+ *       and smaller IQ matrices.  Batched calls also use two f16 planes per
+ *       activation row with one scale, 22 bits of each value and down to 2^-39
+ *       of the row's largest; rows in which a 32-value block is further below it
+ *       than that allows are summed in f32.  Their results are no further from
+ *       exact sums than those of one mi355x_gemv per activation, but they are
+ *       not its bits, and the bits depend on the number of activations),
  *     MI355X_VARIANT_EXACT_F32 (codes -> f32, fp32 FMA; activations used
  *       exactly as given), MI355X_VARIANT_DIGITS (activations as fixed point
  *       per 32-value block -- 20-bit for Q4_0 with int4 dot8 products, 16-bit
- *       for the K/IQ types with int8 dot4 products),
+ *       for the K/IQ types with int8 products -- in batched calls too),
  *     MI355X_VARIANT_GGML_Q8 (the arithmetic of ggml's CPU backend, so that
  *       results follow ggml-cpu rather than the f32 references: Q4_0 -- the
  *       activation row quantized to Q8_0 per 32-value block, integer block

@@ -23,8 +23,8 @@
 // value is more than 2^18 below the row's is wide, and a wavefront sums wide rows
 // in f32 after its tiles, four to a pass over its weights, from the activations
 // as they are.  (us with none, one and all of the rows wide: Q4_0 17408x5120 M =
-// 37 50, 85, 406; IQ3_S 8192x8192 M = 64 48, 75, 458.  Every row's activations go
-// through the vector memory path for 64 weight rows at a time, which bounds it.)
+// 37 48, 84, 403; IQ3_S 8192x8192 M = 64 45, 72, 459.  Every row's activations go
+// through the vector memory path for 64 weight rows at a time.)
 //
 // Work split.  A workgroup of 4 wavefronts computes 256 output columns (weight
 // rows) x 32 or 64 activation rows; a wavefront 64 columns as two 32-wide
@@ -38,12 +38,16 @@
 // superblocks are split over gridDim.y segments whose f32 partials a second
 // kernel adds in segment order.
 //
-// What bounds it.  MFMAs on real data take 19 ns each here (power; 13 ns at
-// full clock); with the decode between them 21 ns, and two (Q6_K, IQ4_XS:
-// three) make one useful product.  On top of that come the weights' loads,
-// where the 64 lanes of a load touch 64 rows.  us per call on MI355X
-// (sequential or 8-row passes before): Q4_0 17408x5120 M = 512 301 (2710),
-// Q6_K 4096x14336 M = 512 218 (6310), Q4_K 14336x4096 M = 37 37 (252).
+// What bounds it (rocprof counters, cycles per SIMD or wavefront).  The matrix and
+// the vector work of a SIMD's two wavefronts hardly overlap: at M = 512 Q6_K
+// 4096x14336 has 172 k cycles of MFMA (32 each; two products, for Q6_K and IQ4_XS
+// three, make one useful one) and 144 k of decode in the 328 k that a wavefront
+// runs, Q4_0 17408x5120 174 k and 165 k in 318 k.  Q4_0 there has 544 workgroups for
+// 512 places, and the last 32 take a round of their own: 292 us against 212.  At M
+// = 37 (Q4_K 14336x4096) a workgroup has two superblocks, 15 k and 17 k cycles of
+// the 45 k that it runs; the staging and the adding launch take 11 of 38 us.  us
+// per call on MI355X (sequential or 8-row passes before): Q4_0 17408x5120 M = 512
+// 293 (2710), Q6_K 4096x14336 M = 512 222 (6310), Q4_K 14336x4096 M = 37 35 (252).
 #include "internal.h"
 #include "kq_device.h"
 #include "q4_0_layout.h"
@@ -194,8 +198,9 @@ __device__ __forceinline__ void store_superblock(const XPlanes &c, int m, int la
 // wavefronts taking the superblocks in turn; the first kPlKeep of each stay in
 // registers between the row's maximum and the conversion.  A row is wide if a
 // block of 32 has a largest scaled value below kWideBelow but not 0: the planes
-// hold a value to 2^-25 at worst, which is then more than 2^-21 of the block's
-// largest (20-bit fixed point: 2^-20), or than 2^-25 where f32 is the measure.
+// hold a value to 2^-25 at worst, which is then at most 2^-21 of the block's
+// largest (the fixed point of the one-row kernels: 2^-18.9 for Q4_0, 2^-16 for the
+// other types), or 2^-25 of it where f32 is the measure.
 constexpr float kWideBelow = 0.0625f, kWideBelowF32 = 1.0f;
 constexpr int kWideRows = 4;
 constexpr int kPlThreads = 1024, kPlWavesG = kPlThreads / 64, kPlKeep = 4;

@@ -14,11 +14,11 @@
 // exact in f32; a block's f32 sums are scaled by its d and added in f32.  An
 // activation with a block whose largest value is more than 2^18 below that of the
 // wavefront's part is wide (the fixed point of the dot-unit forms, with a scale
-// per block, held such a block to 2^-20): after its tiles the workgroup sums wide
+// per block, held such a block to 2^-18.9): after its tiles the workgroup sums wide
 // activations in f32 from their values as they are.  The lanes compare the least
 // that they saw of each activation while they stage it; only where that is small
 // does the workgroup read the activations again to tell.  (us at 8192x8192 M = 8
-// with none, one and all wide 19.8, 48, 95, without the comparison 19.3.)
+// with none, one and all wide 19.8, 47, 97, without the comparison 19.3.)
 //
 // Work split.  A workgroup of 8 wavefronts owns tiles of 16 weight rows and
 // splits K: wavefront v takes QN quads of 4 blocks.  Lane (n, g) = (lane & 15,
@@ -32,9 +32,11 @@
 // quads per wavefront stay in flight; tile sums meet in LDS.  Rows of more than
 // 8192 values go in two launches, the second adding to y.
 //
-// What bounds it.  VALU issue: about 85 instructions per quad and tile and 78
-// per quad to stage the activations, which every workgroup does for itself, so
-// long rows with few tiles per workgroup spend most of their time staging.
+// What bounds it: waiting.  At 8192x8192 M = 8 a wavefront runs 45 k cycles, of
+// which its SIMD issues vector instructions for 16 k (about 85 per quad and tile
+// and 85 per quad to stage the activations) and matrix ones for 2 k (rocprof).
+// Every workgroup reads and converts all activations, 256 KB through each CU's L1
+// there, before its two tiles, with two wavefronts per SIMD to hide it.
 // us per call on MI355X, dot-unit forms -> here: M = 8 8192x8192 25.9 -> 19.8,
 // 4096x4096 11.9 -> 8.3, 17408x5120 42.9 -> 20.0, 151936x2048 73.7 -> 50.
 #include "internal.h"
